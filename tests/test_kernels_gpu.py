@@ -644,6 +644,69 @@ def test_sample_reference_mode_is_softmax_argmax(vsl, orc, dev, H):
     assert dev.get(out)[0] == orc.sample(l, orc.SAMPLE_REFERENCE, 0.7) == 0
 
 
+def _head_logit_cases():
+    """Logit vectors that take each route of the output stage's samplers over its blocks' maxima: few
+    and many blocks, a vocabulary past one pass of the grid, ragged ends, largest logits in one block's
+    rows (a loose bound: more than 256 and more than 1024 candidates), ties, too few finite logits, NaN."""
+    rng = np.random.default_rng(61)
+    cases = {"normal": rng.normal(0, 1.3, 32000), "ragged": rng.normal(0, 1.3, 8195), "wide": rng.normal(0, 1.3, 128256),
+             "one_pass": rng.normal(0, 1.0, 1001), "tiny": rng.normal(0, 1.0, 37), "equal": np.zeros(20000),
+             "integers": rng.integers(0, 3, 16001).astype(float)}
+    packed = rng.normal(0, 1.0, 32000)
+    packed[(np.arange(32000) // 8) % 1024 < 70] += 30.0
+    cases["packed_blocks"] = packed
+    spread = rng.normal(0, 1.0, 32000)
+    spread[(np.arange(32000) // 8) % 1024 % 23 == 3] += 30.0
+    cases["spread_blocks"] = spread
+    inf = np.full(20000, -np.inf)
+    inf[[5, 700, 19999]] = [1.0, 2.0, 2.0]
+    cases["mostly_neg_inf"] = inf
+    nan = rng.normal(0, 1.0, 20000)
+    nan[(np.arange(20000) // 8) % 2 == 0] = np.nan
+    cases["nan_blocks"] = nan
+    near = np.full(32000, -5.0)
+    near[3000] = 1e-6
+    near[1200] = np.nextafter(np.nextafter(np.float32(1e-6), np.float32(0)), np.float32(0))
+    cases["near_tie"] = near
+    cases["all_neg_inf"] = np.full(9000, -np.inf)
+    return {n: v.astype(np.float32) for n, v in cases.items()}
+
+
+@pytest.mark.parametrize("name", list(_head_logit_cases()))
+def test_lm_head_samplers_match_general_path(vsl, orc, dev, H, name):
+    """The output stage's top-k (k up to 128 through the block maxima, past it streaming) and reference
+    samplers draw the token that vsl_sample_logits draws from the same logits, and where no logit is
+    NaN the oracle's.  W holds the logits in its first column and x selects it (no norm), so they are
+    exact; an 8-wave (K > 8192) projection is among the shapes."""
+    l = _head_logit_cases()[name]
+    V = l.size
+    nb = H.vsl_lm_head_ws_blocks()
+    ws_v, ws_i = dev.empty((nb,), np.float32), dev.empty((nb,), np.int32)
+    out = dev.empty((1,), np.int32)
+    dl = dev.put(l)
+    for d in (8, 8200) if name in ("ragged", "one_pass") else (8,):
+        W = np.zeros((V, d), np.float32)
+        W[:, 0] = l
+        x = np.zeros(d, np.float32)
+        x[0] = 1.0
+        dW, dx, logits = dev.put(W), dev.put(x), dev.empty((V,), np.float32)
+        E = dev.put(np.broadcast_to(x, (V, d)).copy())  # every next embedding is x again
+        for mode, T, k in [(2, 0.8, 1), (2, 0.8, 40), (2, 1.3, 64), (2, 1.3, 65), (2, 1.3, 128), (2, 1.3, 129),
+                           (1, 0.7, 1), (1, 1.0, 1)]:
+            toks = dev.empty((4,), np.int32)
+            c = ctrl_buf(vsl, dev, H, 3, max_steps=64, cap=64)
+            smp = vsl.Sampler(mode, T, k, 0, 9)
+            for step in range(4):
+                ok(vsl, H.vsl_lm_head_sample(None, 1e-5, dev.p(dW), 0, V, d, dev.p(dx), dev.p(E), 0, dev.p(logits), smp,
+                                             dev.p(ws_v), dev.p(ws_i), dev.p(toks), dev.p(c), None))
+                ok(vsl, H.vsl_sample_logits(dev.p(dl), V, smp, step, dev.p(out), None))
+                want = int(dev.get(out)[0])
+                assert int(dev.get(toks)[step]) == want, (mode, T, k, step)
+                if not np.isnan(l).any() and (mode == 2 and name != "all_neg_inf" or mode == 1):
+                    assert want == orc.sample(l, mode, T, k, 9, step), (mode, T, k, step)
+            assert np.array_equal(dev.get(logits), l, equal_nan=True)
+
+
 def test_embed_clamps_out_of_range_ids(vsl, dev, H):
     """embedding_lookup.comp:32: an id at or past the vocabulary reads row V - 1 (fp16 and fp32 tables)."""
     V, d = 300, 64

@@ -658,32 +658,31 @@ int gemv_waves_env() {
     return w;
 }
 
+// Waves per block that launch_gemv_k takes for K columns.
+uint32_t gemv_waves_k(uint32_t K) {
+    const int env = gemv_waves_env();
+    if (env == 16 || (env == 8 && K <= kXWideK) || (env == 4 && K <= kWideK)) return (uint32_t)env;
+    return K > kXWideK ? 16u : K > kWideK ? 8u : 4u;
+}
+
 template <class WT, int R, int U, int EPI, class ET = WF32>
 int launch_gemv_k(const GemvArgs& a, uint32_t max_blocks, hipStream_t s) {
-    switch (gemv_waves_env()) {
+    switch (gemv_waves_k(a.K)) {
         case 16: return launch_gemv<WT, R, U, EPI, 16, ET>(a, max_blocks, s);
-        case 8: if (a.K <= kXWideK) return launch_gemv<WT, R, U, EPI, 8, ET>(a, max_blocks, s); break;
-        case 4: if (a.K <= kWideK) return launch_gemv<WT, R, U, EPI, 4, ET>(a, max_blocks, s); break;
-        default: break;
+        case 8: return launch_gemv<WT, R, U, EPI, 8, ET>(a, max_blocks, s);
+        default: return launch_gemv<WT, R, U, EPI, 4, ET>(a, max_blocks, s);
     }
-    if (a.K > kXWideK) return launch_gemv<WT, R, U, EPI, 16, ET>(a, max_blocks, s);
-    return a.K > kWideK ? launch_gemv<WT, R, U, EPI, 8, ET>(a, max_blocks, s)
-                        : launch_gemv<WT, R, U, EPI, 4, ET>(a, max_blocks, s);
 }
 
 template <int R, int EPI>
 uint32_t gemv_blocks_k(uint32_t N, uint32_t K, uint32_t max_blocks) {
     // the grid launch_gemv_k chooses
-    switch (gemv_waves_env()) {
+    switch (gemv_waves_k(K)) {
         case 16: return gemv_blocks<R, EPI, 16>(N, max_blocks);
-        case 8: if (K <= kXWideK) return gemv_blocks<R, EPI, 8>(N, max_blocks); break;
-        case 4: if (K <= kWideK) return gemv_blocks<R, EPI, 4>(N, max_blocks); break;
-        default: break;
+        case 8: return gemv_blocks<R, EPI, 8>(N, max_blocks);
+        default: return gemv_blocks<R, EPI, 4>(N, max_blocks);
     }
-    if (K > kXWideK) return gemv_blocks<R, EPI, 16>(N, max_blocks);
-    return K > kWideK ? gemv_blocks<R, EPI, 8>(N, max_blocks) : gemv_blocks<R, EPI, 4>(N, max_blocks);
 }
-
 
 int check_gemv_shape(uint32_t N, uint32_t K, const char* who) {
     if (N == 0 || K == 0) return vsl_invalid("%s: empty shape", who);
@@ -1798,6 +1797,252 @@ __device__ __forceinline__ uint32_t block_sample(const float* __restrict__ logit
     return s_tok;
 }
 
+// ---------------------------------------------------------------------------------------------
+// samplers over logits whose per-block maxima the output projection left behind
+// ---------------------------------------------------------------------------------------------
+// k_gemv_dec<EPI_ARGMAX> stores the logits and, per block, the largest of its own (ws_val). Block b of
+// nb covers rows i * nb * rpb + b * rpb .. + rpb - 1 for i = 0, 1, ... (rpb rows per pass over the
+// grid), so a value bound on the block maxima names the few rows that can hold what the sampler looks
+// for, and the other blocks' logits are not read again. One block streams logits at ~0.2 cycles each
+// (its outstanding misses bound it), and block_sample streams them two to five times. Output stage,
+// seeded top-k over V = 128256, K = 4096, k = 40: 207.0 -> 178.4 us (163 of them the GEMV); K = 8192,
+// k = 3: 356.9 -> 325.5.
+struct LmBlocks {
+    const float* val;     // per-block maxima; NaN logits never win, a block of NaNs alone holds -inf
+    const float* part;    // reference mode: per-block sums of exp (k_reference_sum)
+    uint32_t nb, n_part;  // nb <= kSampBlock blocks, n_part sums
+    uint32_t rpb_log2;    // log2(rpb)
+};
+constexpr uint32_t kBlockTopK = 128;  // seeded top-k through the block maxima up to this k
+static_assert(kMaxLmBlocks <= (uint32_t)kSampBlock, "one block maximum per sampling thread");
+
+// Calls f(logit, row) for the rows of the lm_head blocks listed in s_blk (n_blk of them, in LDS), eight
+// loads in flight per thread.
+template <class F>
+__device__ __forceinline__ void for_each_block_logit(const float* __restrict__ logits, uint32_t V, const LmBlocks& lb,
+                                                     const uint16_t* s_blk, uint32_t n_blk, uint32_t tid, F&& f) {
+    constexpr int NL = 8;
+    const uint32_t rpb = 1u << lb.rpb_log2, pass = lb.nb << lb.rpb_log2;
+    const uint32_t per = ((V + pass - 1) / pass) << lb.rpb_log2;  // rows per block, the last pass rounded up
+    const uint32_t items = n_blk * per;
+    for (uint32_t base = 0; base < items; base += kSampBlock * NL) {
+        float v[NL];
+        uint32_t row[NL];
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            const uint32_t t = base + tid + (uint32_t)j * kSampBlock;
+            row[j] = 0xFFFFFFFFu;
+            if (t < items) {
+                const uint32_t b = t / per, r = t - b * per;
+                row[j] = (r >> lb.rpb_log2) * pass + ((uint32_t)s_blk[b] << lb.rpb_log2) + (r & (rpb - 1));
+            }
+            v[j] = row[j] < V ? logits[row[j]] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < NL; ++j)
+            if (row[j] < V) f(v[j], row[j]);
+    }
+}
+
+// Seeded top-k (Utils.cpp:151-171) for k <= kBlockTopK, exactly the candidates and the arithmetic of
+// block_sample. tau, the k-th largest of the maxima of 128 (k > 64: 256) groups of adjacent blocks, has
+// k distinct logits at or above it, so every logit of the top k is >= tau and lies in a block whose
+// maximum is (about k blocks; at V = 128256, k = 40: 5000 of the logits). The few candidates (about
+// k, for ordinary logits) are ranked by counting, each of the 1024 threads comparing one of them
+// with a share of the others. Returns false, having drawn nothing, where the bound does not help: fewer
+// than k groups hold a number above -inf, or more than kSampBlock logits reach tau.
+__device__ bool topk_sample_blocks(const float* __restrict__ logits, uint32_t V, const LmBlocks& lb, uint32_t k,
+                                   float temperature, uint32_t k0, uint32_t k1, uint64_t step, uint64_t* s_cand,
+                                   uint64_t* s_sort, uint32_t& tok) {
+    __shared__ uint32_t s_gmax[256], s_gt[256], s_ge[256];
+    __shared__ uint64_t s_topk[kBlockTopK];
+    __shared__ uint16_t s_blk[kSampBlock];
+    __shared__ uint32_t s_nblk, s_n, s_tau32, s_out;
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t bkey = tid < lb.nb ? value_key(lb.val[tid]) : 0u;
+    const uint32_t ng = k <= 64 ? 128u : 256u;
+    uint32_t gm = bkey;  // the group's maximum: four adjacent lanes, then the other four of the half row
+    auto dpp_max = [](uint32_t v, uint32_t o) { return o > v ? o : v; };
+    gm = dpp_max(gm, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gm, 0xB1, 0xF, 0xF, false));
+    gm = dpp_max(gm, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gm, 0x4E, 0xF, 0xF, false));
+    if (k <= 64) gm = dpp_max(gm, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gm, 0x141, 0xF, 0xF, false));
+    const uint32_t per_group = kSampBlock / ng;
+    if (tid % per_group == 0) s_gmax[tid / per_group] = gm;
+    if (tid < 256) {
+        s_gt[tid] = 0;
+        s_ge[tid] = 0;
+    }
+    if (tid == 0) {
+        s_nblk = 0;
+        s_n = 0;
+    }
+    __syncthreads();
+    // thread (j, p): key j against share p of the keys
+    const uint32_t j = tid & (ng - 1), share = ng * ng / kSampBlock, p0 = tid / ng * share;
+    {
+        const uint32_t mine = s_gmax[j];
+        uint32_t gt = 0, ge = 0;
+        for (uint32_t i = 0; i < share; ++i) {
+            const uint32_t o = s_gmax[p0 + i];
+            gt += o > mine;
+            ge += o >= mine;
+        }
+        atomicAdd(&s_gt[j], gt);
+        atomicAdd(&s_ge[j], ge);
+    }
+    __syncthreads();
+    if (tid < ng && s_gt[tid] < k && s_ge[tid] >= k) s_tau32 = s_gmax[tid];  // equal keys store the same value
+    __syncthreads();
+    const uint32_t tau = s_tau32;
+    if (tau <= value_key(-INFINITY)) return false;
+    if (bkey >= tau) s_blk[atomicAdd(&s_nblk, 1u)] = (uint16_t)tid;
+    if (tid < 256) s_gt[tid] = 0;
+    __syncthreads();
+    for_each_block_logit(logits, V, lb, s_blk, s_nblk, tid, [&](float l, uint32_t i) {
+        const uint32_t vk = value_key(l);
+        if (vk >= tau) {
+            const uint32_t slot = atomicAdd(&s_n, 1u);
+            if (slot < (uint32_t)kSampBlock) s_cand[slot] = rank_key(vk, i);
+        }
+    });
+    __syncthreads();
+    const uint32_t n = s_n;  // >= k
+    if (n > (uint32_t)kSampBlock) return false;
+    if (n <= 256) {
+        const uint32_t nr = n <= 128 ? 128u : 256u;
+        if (tid >= n && tid < nr) s_cand[tid] = 0ull;  // ranks after every logit's key
+        __syncthreads();
+        const uint32_t c = tid & (nr - 1), sh = nr * nr / kSampBlock, q0 = tid / nr * sh;
+        const uint64_t mine = s_cand[c];
+        uint32_t gt = 0;
+        for (uint32_t i = 0; i < sh; ++i) gt += s_cand[q0 + i] > mine;
+        atomicAdd(&s_gt[c], gt);
+        __syncthreads();
+        if (tid < n && s_gt[tid] < k) s_topk[s_gt[tid]] = s_cand[tid];
+    } else {
+        uint64_t x = tid < n ? s_cand[tid] : 0ull;
+        x = bitonic_desc<kSampBlock>(x, tid, s_sort);
+        if (tid < k) s_topk[tid] = x;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        // weights exp((l_i - max) / T) / sum, two per lane, summed and walked in rank order as in
+        // block_sample
+        const float mx = key_value((uint32_t)(s_topk[0] >> 32));
+        float e[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t i = lane + 64 * h;
+            e[h] = i < k ? expf((key_value((uint32_t)(s_topk[i < k ? i : 0] >> 32)) - mx) / temperature) : 0.f;
+        }
+        float sum = 0.f;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            if (k > 64u * h) {
+#pragma unroll
+                for (int i = 0; i < 64; ++i)
+                    if (64u * h + i < k) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e[h]), i));
+            }
+        const float r = sample_uniform(k0, k1, step);
+        float cum = 0.f;
+        uint32_t pick = 0;
+        bool found = false;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int w = __float_as_int(e[h] / sum);
+            if (k > 64u * h && !found) {
+#pragma unroll
+                for (int i = 0; i < 64; ++i) {
+                    if (64u * h + i < k && !found) {
+                        cum += __int_as_float(__builtin_amdgcn_readlane(w, i));
+                        if (r < cum) { pick = 64 * h + i; found = true; }
+                    }
+                }
+            }
+        }
+        if (lane == 0) s_out = ~(uint32_t)s_topk[pick];
+    }
+    __syncthreads();
+    tok = s_out;
+    return true;
+}
+
+// Reference mode, first launch: sums of exp(l / T - max) over slices of the logits, one per block (one
+// block over V = 128256 logits is bound by its expf arithmetic and its misses; 256 blocks share them).
+// The maximum of l / T is that of the block maxima divided by T: a division by T > 0 keeps order.
+constexpr uint32_t kRefBlocks = 256;
+constexpr int kRefThreads = 256;
+static_assert(kRefBlocks <= kMaxLmBlocks, "the sums take the place of the block indices");
+__device__ __forceinline__ float ref_scaled(float l, float temperature) { return temperature != 1.0f ? l / temperature : l; }
+
+__global__ __launch_bounds__(kRefThreads) void k_reference_sum(const float* __restrict__ logits, uint32_t V, float T,
+                                                               const float* __restrict__ ws_val, uint32_t nb,
+                                                               float* __restrict__ part, const vsl_ctrl* ctrl) {
+    __shared__ float red[kRefThreads / 64];
+    if (ctrl->done) return;
+    const uint32_t tid = threadIdx.x;
+    float mx = -INFINITY;
+    for (uint32_t b = tid; b < nb; b += kRefThreads) mx = fmaxf(mx, ref_scaled(ws_val[b], T));
+    mx = wave_max_dpp(mx);
+    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    __syncthreads();
+    for (int w = 0; w < kRefThreads / 64; ++w) mx = fmaxf(mx, red[w]);
+    __syncthreads();
+    float sum = 0.f;
+    for (uint32_t i = blockIdx.x * kRefThreads + tid; i < V; i += kRefBlocks * kRefThreads)
+        sum += expf(ref_scaled(logits[i], T) - mx);
+    sum = wave_sum_dpp(sum);
+    if ((tid & 63) == 0) red[tid >> 6] = sum;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < kRefThreads / 64; ++w) sum += red[w];
+        part[blockIdx.x] = sum;
+    }
+}
+
+// Reference mode, second launch (see block_sample): the first index of the largest exp(l / T - max) /
+// sum. Only logits within kRefNear of the maximum can round to its probability (exp(-kRefNear) is 1e-2
+// below 1), so only blocks whose maximum is that near are read.
+constexpr float kRefNear = 0.01f;
+__device__ uint32_t reference_sample_blocks(const float* __restrict__ logits, uint32_t V, const LmBlocks& lb,
+                                            float temperature) {
+    __shared__ float s_f[kSampBlock / 64];
+    __shared__ uint32_t s_i[kSampBlock / 64];
+    __shared__ uint16_t s_blk[kSampBlock];
+    __shared__ uint32_t s_nblk, s_pick;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const float bv = tid < lb.nb ? ref_scaled(lb.val[tid], temperature) : -INFINITY;
+    float mx = wave_max_dpp(bv);
+    if (lane == 0) s_f[wave] = mx;
+    if (tid == 0) s_nblk = 0;
+    __syncthreads();
+    mx = s_f[0];
+    for (int w = 1; w < kSampBlock / 64; ++w) mx = fmaxf(mx, s_f[w]);
+    __syncthreads();
+    float sum = tid < lb.n_part ? lb.part[tid] : 0.f;
+    sum = wave_sum_dpp(sum);
+    if (lane == 0) s_f[wave] = sum;
+    if (bv - mx >= -kRefNear) s_blk[atomicAdd(&s_nblk, 1u)] = (uint16_t)tid;  // nb > 0: none only with a NaN sum
+    __syncthreads();
+    sum = 0.f;
+    for (int w = 0; w < kSampBlock / 64; ++w) sum += s_f[w];
+    float best = -INFINITY;
+    uint32_t bi = 0xFFFFFFFFu;
+    for_each_block_logit(logits, V, lb, s_blk, s_nblk, tid, [&](float l, uint32_t i) {
+        argmax_merge(best, bi, expf(ref_scaled(l, temperature) - mx) / sum, i);
+    });
+    wave_argmax(best, bi);
+    __syncthreads();
+    if (lane == 0) { s_f[wave] = best; s_i[wave] = bi; }
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < kSampBlock / 64; ++w) argmax_merge(best, bi, s_f[w], s_i[w]);
+        s_pick = bi == 0xFFFFFFFFu ? 0u : bi;  // every probability NaN: token 0
+    }
+    __syncthreads();
+    return s_pick;
+}
+
 __global__ __launch_bounds__(kSampBlock) void k_sample_logits(const float* logits, uint32_t V, int mode, float T,
                                                               uint32_t top_k, uint32_t k0, uint32_t k1, uint64_t step,
                                                               uint32_t* out) {
@@ -1808,10 +2053,19 @@ __global__ __launch_bounds__(kSampBlock) void k_sample_logits(const float* logit
 template <class ET>
 __global__ __launch_bounds__(kSampBlock) void k_sample_finish(const float* logits, uint32_t V, uint32_t d, int mode,
                                                               float T, uint32_t top_k, uint32_t k0, uint32_t k1,
-                                                              const void* embed, float* x_next, uint32_t* tokens,
-                                                              vsl_ctrl* ctrl) {
+                                                              LmBlocks lb, const void* embed, float* x_next,
+                                                              uint32_t* tokens, vsl_ctrl* ctrl) {
+    __shared__ uint64_t s_cand[kSampBlock];
+    __shared__ uint64_t s_sort[kSampBlock];
     if (ctrl->done) return;
-    const uint32_t tok = block_sample(logits, V, mode, T, top_k, k0, k1, ctrl->step);
+    uint32_t tok;
+    if (mode == VSL_SAMPLE_REFERENCE) {
+        tok = reference_sample_blocks(logits, V, lb, T);
+    } else {
+        const uint32_t k = top_k > V ? V : top_k;
+        if (k > kBlockTopK || !topk_sample_blocks(logits, V, lb, k, T, k0, k1, ctrl->step, s_cand, s_sort, tok))
+            tok = block_sample(logits, V, mode, T, top_k, k0, k1, ctrl->step);
+    }
     finish_token<ET>(tok, V, d, embed, x_next, tokens, ctrl);
 }
 
@@ -2753,10 +3007,9 @@ extern "C" int vsl_lm_head_sample(const float* gamma, float eps, const void* W, 
     a.W = W; a.N = V; a.K = d; a.x = x; a.gamma = gamma; a.eps = eps; a.y = logits;
     a.ws_val = ws_val; a.ws_idx = ws_idx; a.tokens = tokens; a.embed = embed; a.x_next = x;
     a.ctrl = ctrl;
+    if (int rc = launch_gemv_w<2, EPI_ARGMAX>(wdtype, a, kMaxLmBlocks, s, "vsl_lm_head_sample")) return rc;
+    const uint32_t nb = gemv_blocks_k<2, EPI_ARGMAX>(V, d, kMaxLmBlocks);
     if (fused) {
-        int rc = launch_gemv_w<2, EPI_ARGMAX>(wdtype, a, kMaxLmBlocks, s, "vsl_lm_head_sample");
-        if (rc) return rc;
-        const uint32_t nb = gemv_blocks_k<2, EPI_ARGMAX>(V, d, kMaxLmBlocks);
         if (embed_dtype == VSL_DT_F16)
             k_argmax_finish<WF16><<<1, kFinishThreads, 0, s>>>(ws_val, ws_idx, nb, V, d, embed, x, tokens, ctrl);
         else
@@ -2764,16 +3017,21 @@ extern "C" int vsl_lm_head_sample(const float* gamma, float eps, const void* W, 
         HIP_TRY(hipGetLastError());
         return VSL_OK;
     }
-    // logits only (EPI_STORE with the norm prologue), then the sampling kernel
-    int rc = launch_gemv_w<2, EPI_STORE>(wdtype, a, 1u << 20, s, "vsl_lm_head_sample");
-    if (rc) return rc;
+    // the sampling kernel reads the block maxima first and then the blocks that matter
     const uint64_t key = vsl_derive_key(sampler.seed, "sampler");
+    float* part = reinterpret_cast<float*>(ws_idx);
+    LmBlocks lb{ws_val, part, nb, kRefBlocks, 0};
+    while ((1u << lb.rpb_log2) < 2 * gemv_waves_k(d)) ++lb.rpb_log2;  // two rows per wave
+    if (sampler.mode == VSL_SAMPLE_REFERENCE) {
+        k_reference_sum<<<kRefBlocks, kRefThreads, 0, s>>>(logits, V, sampler.temperature, ws_val, nb, part, ctrl);
+        HIP_TRY(hipGetLastError());
+    }
     if (embed_dtype == VSL_DT_F16)
         k_sample_finish<WF16><<<1, kSampBlock, 0, s>>>(logits, V, d, sampler.mode, sampler.temperature, sampler.top_k,
-                                                       (uint32_t)key, (uint32_t)(key >> 32), embed, x, tokens, ctrl);
+                                                       (uint32_t)key, (uint32_t)(key >> 32), lb, embed, x, tokens, ctrl);
     else
         k_sample_finish<WF32><<<1, kSampBlock, 0, s>>>(logits, V, d, sampler.mode, sampler.temperature, sampler.top_k,
-                                                       (uint32_t)key, (uint32_t)(key >> 32), embed, x, tokens, ctrl);
+                                                       (uint32_t)key, (uint32_t)(key >> 32), lb, embed, x, tokens, ctrl);
     HIP_TRY(hipGetLastError());
     return VSL_OK;
 }
