@@ -125,6 +125,32 @@ def test_gemv_batched_rows(vsl, orc, dev, H, N, K, B, ydt):
         assert np.all(np.abs(y - ref) <= np.abs(ref) * 2.0 ** -11 + 1e-4 * np.max(np.abs(ref)))
 
 
+@pytest.mark.parametrize("N,K,B,ydt,off", [
+    (1, 512, 2, 0, 0),         # one row; eight units for the 16-wave blocks
+    (300, 1536, 5, 1, 0),      # a ragged last fragment, odd B
+    (6143, 2048, 16, 0, 0),    # the largest N of one fragment per block
+    (6144, 512, 3, 1, 0), (12271, 1024, 7, 0, 0),     # two fragments: one unit per wave; ragged end
+    (12272, 512, 16, 0, 0), (14337, 1536, 9, 1, 0),   # four fragments: two units; six; ragged end
+    (1000, 14336, 4, 0, 0),    # fourteen units per wave
+    (500, 1024, 6, 0, 1),      # X not 16-byte aligned: the gathering kernel
+])
+def test_gemv_row_major(vsl, dev, H, N, K, B, ydt, off):
+    """vsl_gemv on fp16 row-major X, B columns, at the edges of its block shapes and units per wave,
+    against the fp64 product; nothing past Y's N * B values is written."""
+    rng = np.random.default_rng(N + K + B)
+    W = rng.normal(0, 0.02, (N, K)).astype(np.float16)
+    X = rng.normal(0, 1, (K, B)).astype(np.float16)
+    dX = dev.put(np.concatenate([np.zeros(off, np.float16), X.ravel()]))
+    yt = np.float32 if ydt == 0 else np.float16
+    Y = dev.put(np.full(N * B + 8, 7.0, yt))
+    ok(vsl, H.vsl_gemv(dev.p(dev.put(W)), 1, N, K, dev.p(dX) + 2 * off, 1, B, dev.p(Y), ydt, None))
+    y = dev.get(Y)
+    assert np.all(y[N * B:] == 7.0)
+    ref = W.astype(np.float64) @ X.astype(np.float64)
+    # fp32 accumulation of exact products: about sqrt(K) ulps; fp16 results one rounding
+    assert rel_err(y[:N * B].reshape(N, B).astype(np.float64), ref) < (1e-5 if ydt == 0 else 2.0 ** -10)
+
+
 @pytest.mark.parametrize("B,off", [(1, 1), (1, 4), (4, 1), (12, 3)])
 def test_gemv_batched_x_offset(vsl, orc, dev, H, B, off):
     """X starting `off` halfs past an aligned address: B = 1 takes the decode GEMV (8-byte X loads) only

@@ -51,3 +51,7 @@ void vsl_gemm_splitk_partials(uint32_t ksplit, void* stream, const void* A, cons
                               uint32_t K, int am, float* ws, int b8s);
 int vsl_gemm_splitk_launch(uint32_t ksplit, void* stream, const void* A, const void* B, uint32_t M, uint32_t N,
                            uint32_t K, void* C, int epi, int am, float* ws, int b8s);
+
+// The skinny product of vsl_gemv on row-major X (vsl_skinny.hip): fp16 W and X, K % 64 == 0, X 16-byte
+// aligned, 2 <= B <= 16.
+void vsl_skinny_rows(const void* W, uint32_t N, uint32_t K, const void* X, uint32_t B, void* Y, bool y16, void* stream);
