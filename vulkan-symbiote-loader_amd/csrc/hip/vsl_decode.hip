@@ -1805,7 +1805,7 @@ __device__ __forceinline__ uint32_t block_sample(const float* __restrict__ logit
 // grid), so a value bound on the block maxima names the few rows that can hold what the sampler looks
 // for, and the other blocks' logits are not read again. One block streams logits at ~0.2 cycles each
 // (its outstanding misses bound it), and block_sample streams them two to five times. Output stage,
-// seeded top-k over V = 128256, K = 4096, k = 40: 207.0 -> 178.4 us (163 of them the GEMV); K = 8192,
+// seeded top-k over V = 128256, K = 4096, k = 40: 207.0 -> 176.9 us (163 of them the GEMV); K = 8192,
 // k = 3: 356.9 -> 325.5.
 struct LmBlocks {
     const float* val;     // per-block maxima; NaN logits never win, a block of NaNs alone holds -inf
@@ -1935,29 +1935,20 @@ __device__ bool topk_sample_blocks(const float* __restrict__ logits, uint32_t V,
             const uint32_t i = lane + 64 * h;
             e[h] = i < k ? expf((key_value((uint32_t)(s_topk[i < k ? i : 0] >> 32)) - mx) / temperature) : 0.f;
         }
+        // (loops, not unrolled code: the launch runs once per token, its instructions come from memory)
+        const uint32_t n0 = k < 64 ? k : 64;
         float sum = 0.f;
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-            if (k > 64u * h) {
-#pragma unroll
-                for (int i = 0; i < 64; ++i)
-                    if (64u * h + i < k) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e[h]), i));
-            }
+        for (uint32_t i = 0; i < n0; ++i) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e[0]), i));
+        for (uint32_t i = 64; i < k; ++i) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e[1]), i - 64));
         const float r = sample_uniform(k0, k1, step);
+        const int w0 = __float_as_int(e[0] / sum), w1 = __float_as_int(e[1] / sum);
         float cum = 0.f;
         uint32_t pick = 0;
-        bool found = false;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int w = __float_as_int(e[h] / sum);
-            if (k > 64u * h && !found) {
-#pragma unroll
-                for (int i = 0; i < 64; ++i) {
-                    if (64u * h + i < k && !found) {
-                        cum += __int_as_float(__builtin_amdgcn_readlane(w, i));
-                        if (r < cum) { pick = 64 * h + i; found = true; }
-                    }
-                }
+        for (uint32_t i = 0; i < k; ++i) {
+            cum += __int_as_float(__builtin_amdgcn_readlane(i < 64 ? w0 : w1, i & 63));
+            if (r < cum) {
+                pick = i;
+                break;
             }
         }
         if (lane == 0) s_out = ~(uint32_t)s_topk[pick];
