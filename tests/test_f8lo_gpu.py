@@ -222,6 +222,75 @@ def test_gemm_f8lo_splitk(vsl, dev, H, M, N, K, epi):
             assert rel_err(out - (C0[rows] if epi == 2 else 0.0), ref) < 5e-6
 
 
+@pytest.mark.parametrize("M,N,K,epi,amode,cmode", [
+    (1, 6144, 512, 0, "x2", None),      # 96 weight rows per block, two chunks, one unit per wave
+    (3, 6144, 4096, 0, "f8", None),     # 8B QKV
+    (17, 2048, 2048, 2, "x2", None),    # 64 weight rows per block, residual add
+    (45, 4096, 4096, 2, "f8", None),    # 8B O projection: 128 weight rows per block
+    (64, 4096, 14336, 2, "x2", None),   # 8B down projection, seven units per wave
+    (33, 2048, 8192, 1, "x2", None),    # fp16 store
+    (16, 8192, 768, 0, "x2", None),     # chunks of six units: waves of one and two
+    (48, 8192, 1280, 0, "f8", None),    # chunks of ten units: waves of two and three
+    (2, 14336, 256, 3, "x2", "x2"),     # SwiGLU: 112 weight rows per block, one unit per wave
+    (45, 14336, 4096, 3, "x2", "x2"),   # 8B gate/up
+    (64, 8192, 2048, 3, "x2", "x2"),    # 1B gate/up: 64 weight rows per block
+    (40, 28672, 1024, 3, "f8", "f8"),   # the 70B-class width
+    (31, 8192, 384, 3, "f8", "x2"),     # waves of one and two units
+    (20, 1984, 640, 3, "x2", "f16"),    # an odd multiple of 64 outputs
+    (97, 3072, 2048, 0, "x2", None),    # two row blocks: 1B QKV and down projection, ragged and whole
+    (128, 2048, 8192, 2, "x2", None),
+    (65, 8192, 2048, 3, "x2", "x2"), (128, 8192, 2048, 3, "x2", "x2"),
+    (30, 768, 2048, 2, "x2", None),     # too narrow for a K split: 16 weight rows per block
+    (5, 1280, 768, 0, "x2", None), (100, 768, 768, 1, "x2", None), (64, 256, 256, 2, "f8", None),
+])
+def test_gemm_few_rows(vsl, dev, H, M, N, K, epi, amode, cmode):
+    """Chunks of up to 128 rows on the few-row kernel: every row tile count, block width, chunk count and
+    units-per-wave remainder, against the fp64 product of the carried activations with the fp16 weights
+    (an F16F8 lo plane is widened exactly, so the weights are not rounded to e4m3 here)."""
+    rng = np.random.default_rng(M + N + K + epi)
+    nb = 2 * N if epi == 3 else N
+    A = rng.normal(0, 1, (M, K)).astype(np.float32)
+    B = rng.normal(0, 0.02, (nb, K)).astype(np.float16)
+    if amode == "f8":
+        dA, hi, val = f8_buffer(dev, A)
+    else:
+        hi = A.astype(np.float16)
+        lo = (A - hi.astype(np.float32)).astype(np.float16)
+        dA, val = dev.put(np.concatenate([hi, lo])), hi.astype(np.float64) + lo.astype(np.float64)
+    prod = val @ B.astype(np.float64).T
+    flags = epi | (vsl.GEMM_A_F8 if amode == "f8" else vsl.GEMM_A_X2)
+    if epi == 3:
+        flags |= {"f8": vsl.GEMM_C_F8, "x2": vsl.GEMM_C_X2, "f16": 0}[cmode]
+        C = dev.put(np.full((4 * M * N,), 0x7E, np.uint8))
+        ok(vsl, H.vsl_gemm_f16(dev.p(dA), dev.p(dev.put(B)), M, N, K, dev.p(C), flags, None))
+        ref = prod[:, :N] / (1.0 + np.exp(-prod[:, :N])) * prod[:, N:]
+        flat = dev.get(C).reshape(-1).view(np.uint8)
+        hi_o = flat[:2 * M * N].view(np.float16).reshape(M, N)
+        if cmode == "f8":
+            assert rel_err(T.f16f8_value(hi_o, flat[2 * M * N:3 * M * N].reshape(M, N)), ref) < 2.0 ** -15
+            used = 3
+        elif cmode == "x2":
+            o = flat.view(np.float16).reshape(2, M, N).astype(np.float64)
+            assert rel_err(o[0] + o[1], ref) < 2e-6
+            used = 4
+        else:
+            assert rel_err(hi_o.astype(np.float64), ref) < 2.0 ** -10
+            used = 2
+        assert np.all(flat[used * M * N:] == 0x7E)
+        return
+    need = H.vsl_gemm_f16_ws_bytes(M, N, K, flags)
+    assert (need > 0) == (N > 1280)
+    ws = dev.empty((max(need // 4, 4),), np.float32)
+    C0 = rng.normal(0, 1, (M, N)).astype(np.float32) if epi == 2 else np.zeros((M, N), np.float32)
+    C = dev.empty((M, N), np.float16) if epi == 1 else dev.put(C0)
+    ok(vsl, H.vsl_gemm_f16_ws(dev.p(dA), dev.p(dev.put(B)), M, N, K, dev.p(C), flags, dev.p(ws), need, None))
+    out = dev.get(C).astype(np.float64)
+    if epi == 1:
+        assert rel_err(out, prod) < 2.0 ** -10
+    else:
+        assert rel_err(out - (C0 if epi == 2 else 0.0), prod) < 5e-6
+
+
 @pytest.mark.parametrize("n,off", [(1, 0), (7, 0), (8, 0), (1000, 1), (4097, 3), (1 << 20, 0), ((1 << 20) + 5, 8)])
 def test_absmax_f16(vsl, dev, H, n, off):
     """vsl_absmax_f16: the largest finite |x| (infinities and NaN skipped) over any length and start

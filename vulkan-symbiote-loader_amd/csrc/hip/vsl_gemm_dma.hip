@@ -628,6 +628,7 @@ static bool splitk_narrow(uint32_t M, uint32_t N, uint32_t ksplit) {
 
 void vsl_gemm_splitk_partials(uint32_t ksplit, void* stream, const void* A, const void* B, uint32_t M, uint32_t N,
                               uint32_t K, int am, float* ws, int b8s) {
+    if (vsl_gemm_rows_partials(ksplit, stream, A, B, M, N, K, am, ws)) return;
     const B8Shift b8 = b8_shift(b8s);
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const vsl_half* a = static_cast<const vsl_half*>(A);

@@ -52,6 +52,18 @@ void vsl_gemm_splitk_partials(uint32_t ksplit, void* stream, const void* A, cons
 int vsl_gemm_splitk_launch(uint32_t ksplit, void* stream, const void* A, const void* B, uint32_t M, uint32_t N,
                            uint32_t K, void* C, int epi, int am, float* ws, int b8s);
 
+// Few-row prompt GEMM (vsl_gemm_rows.hip), split-A forms: kGemmAX2 up to kRowsMaxM rows, kGemmAF8 up to
+// kRowsMaxM8.
+constexpr uint32_t kRowsMaxM = 128, kRowsMaxM8 = 64;
+// The K split its partials take, at most max_ks (0: the shape or form is not served).
+uint32_t vsl_gemm_rows_split(uint32_t M, uint32_t N, uint32_t K, int am, uint32_t max_ks);
+// As vsl_gemm_splitk_partials; false (nothing launched) when the form or shape is not served at ks.
+bool vsl_gemm_rows_partials(uint32_t ks, void* stream, const void* A, const void* B, uint32_t M, uint32_t N, uint32_t K,
+                            int am, float* ws);
+// As vsl_gemm_dma_launch, without a K split; false (nothing launched) when not served.
+bool vsl_gemm_rows_direct(void* stream, const void* A, const void* B, uint32_t M, uint32_t N, uint32_t K, void* C, int epi,
+                          int am, int cm);
+
 // The skinny product of vsl_gemv on row-major X (vsl_skinny.hip): fp16 W and X, K % 64 == 0, X 16-byte
 // aligned, 2 <= B <= 16.
 void vsl_skinny_rows(const void* W, uint32_t N, uint32_t K, const void* X, uint32_t B, void* Y, bool y16, void* stream);

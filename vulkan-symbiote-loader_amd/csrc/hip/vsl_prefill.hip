@@ -817,6 +817,7 @@ static uint32_t gemm_tiles(uint32_t M, uint32_t N) {
 }
 
 constexpr uint32_t kDmaMinTiles = 192;
+constexpr uint32_t kRowsNarrowN = 8192;  // a block per 16 weight rows: up to two per CU
 
 // A operand form of a GEMM's flags (the caller has rejected A_X2 | A_F8 together)
 static int gemm_a_mode(int flags) {
@@ -840,14 +841,17 @@ static bool a_flags_valid(int a_flags, int* shift) {
            gemm_b8_shift(a_flags, shift);
 }
 
-// The K split launch_gemm takes for a shape and workspace (0: unsplit kernels).
-static uint32_t splitk_choice(uint32_t M, uint32_t N, uint32_t K, int epi, const float* ws, uint64_t ws_bytes) {
+// The K split launch_gemm takes for a shape, A form and workspace (0: unsplit kernels). Few rows of a
+// split A take the few-row kernel's split, at most the plan's (so the workspace holds it).
+static uint32_t splitk_choice(uint32_t M, uint32_t N, uint32_t K, int epi, int am, const float* ws, uint64_t ws_bytes) {
     for (int cfg = 0; cfg < 2; ++cfg)
         if (vsl_gemm_dma_tiles(cfg, M, N, K, epi) >= kDmaMinTiles) return 0;
     if (!ws) return 0;
     uint64_t need = 0;
     const uint32_t ks = vsl_gemm_splitk_plan(M, N, K, epi, kDmaMinTiles, &need);
-    return ks && need <= ws_bytes ? ks : 0;
+    if (!ks || need > ws_bytes) return 0;
+    const uint32_t rows = vsl_gemm_rows_split(M, N, K, am, ks);
+    return rows ? rows : ks;
 }
 
 static bool aligned_to(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
@@ -857,6 +861,13 @@ template <int EPI>
 static int launch_gemm(hipStream_t s, const vsl_half* a, const vsl_half* b, uint32_t M, uint32_t N, uint32_t K,
                        void* C, int am, int cm, float* ws, uint64_t ws_bytes, int b8s) {
     auto blocks = [](uint32_t tiles) { return ((tiles + 7) / 8) * 8; };  // whole XCD ranges (tile_of)
+    // few rows of a split A: the SwiGLU product streams its weights once (the fp8 forms on the shapes that
+    // the direct-to-LDS tiles take)
+    if constexpr (EPI == VSL_EPI_SWIGLU) {
+        if (((am != kGemmAF8 && cm != kGemmCF8) || vsl_gemm_dma_tiles(1, M, N, K, EPI)) &&
+            vsl_gemm_rows_direct(s, a, b, M, N, K, C, EPI, am, cm))
+            return VSL_OK;
+    }
     // shapes whose 256 x 256 (else 128 x 256) tiles cover at least three quarters of the CUs take
     // the direct-to-LDS kernel
     for (int cfg = 0; cfg < 2; ++cfg)
@@ -865,11 +876,15 @@ static int launch_gemm(hipStream_t s, const vsl_half* a, const vsl_half* b, uint
                        ? VSL_OK
                        : vsl_invalid("vsl_gemm_f16: shape %ux%ux%u does not fit the direct-to-LDS tiles", M, N, K);
     // otherwise, with a workspace, split K over enough blocks
-    if (const uint32_t ks = splitk_choice(M, N, K, EPI, ws, ws_bytes)) {
+    if (const uint32_t ks = splitk_choice(M, N, K, EPI, am, ws, ws_bytes)) {
         if (vsl_gemm_splitk_launch(ks, s, a, b, M, N, K, C, EPI, am, ws, b8s))
             return vsl_invalid("vsl_gemm_f16: split-K epilogue %d", EPI);
         return VSL_OK;
     }
+    // narrow shapes of few rows that no split serves: a block per 16 weight rows
+    if (EPI != VSL_EPI_SWIGLU && N <= kRowsNarrowN && (am != kGemmAF8 || vsl_gemm_dma_tiles(1, M, N, K, EPI)) &&
+        vsl_gemm_rows_direct(s, a, b, M, N, K, C, EPI, am, cm))
+        return VSL_OK;
     // the fp8 lo forms exist in the direct-to-LDS kernel only: on shapes its 128 x 256 tiles take, its
     // 64 x 128 tiles where those cover the CUs (no workspace: O of a 512-row chunk 94 -> 56 us with its
     // RMSNorm), else its larger tiles even when they leave CUs idle
@@ -1042,7 +1057,7 @@ extern "C" int vsl_gemm_f16_qkv_rope_append(const void* A, const void* Wqkv, uin
     const uint32_t N = (n_q + 2 * n_kv) * hd;
     float* ws = static_cast<float*>(workspace);
     const bool x2 = q_dtype == VSL_DT_F16X2, kv32 = kv_dtype == VSL_DT_F32;
-    const uint32_t ks = splitk_choice(S, N, K, VSL_EPI_STORE_F32, ws, ws ? ws_bytes : 0);
+    const uint32_t ks = splitk_choice(S, N, K, VSL_EPI_STORE_F32, gemm_a_mode(a_flags), ws, ws ? ws_bytes : 0);
     if (ks && rope_split4_fits(ws, hd, rope_cos, rope_sin, q_out, kcache, vcache, kv32)) {
         hipStream_t s = static_cast<hipStream_t>(stream);
         vsl_half* qo = static_cast<vsl_half*>(q_out);
@@ -1097,7 +1112,7 @@ extern "C" int vsl_gemm_f16_resid_rmsnorm(const void* A, const void* B, uint32_t
     if (workspace && !aligned_to(workspace, 16)) return vsl_invalid("%s: workspace must be 16-byte aligned", fn);
     if (M == 0) return VSL_OK;
     float* ws = static_cast<float*>(workspace);
-    const uint32_t ks = splitk_choice(M, N, K, VSL_EPI_RESID, ws, ws ? ws_bytes : 0);
+    const uint32_t ks = splitk_choice(M, N, K, VSL_EPI_RESID, gemm_a_mode(a_flags), ws, ws ? ws_bytes : 0);
     const uint32_t nv = N / 1024;
     // (the unrolled sums hold up to 32 float4 of partials per thread; more than 8 partials take the
     // loop of the runtime-count variant)
