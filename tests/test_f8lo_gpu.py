@@ -187,6 +187,34 @@ def test_gemm_f8lo_tiles(vsl, dev, H, M, N, K, epi, cmode):
             assert rel_err(out - base, exact) < 2.0 ** -13
 
 
+@pytest.mark.parametrize("M,N,K,amode", [
+    (700, 14336, 256, "f8"),    # 85 columns of 256 x 256 tiles, 27 of 128 x 256
+    (1100, 14336, 256, "x2"),   # 102 and 10; a ragged last row tile in both
+    (1300, 8192, 384, "f8"),    # 42 and 22; an odd number of 128-column stage groups
+])
+def test_gemm_mixed_rounds(vsl, dev, H, M, N, K, amode):
+    """SwiGLU products whose last round of 256 x 256 tiles would be less than half full run its columns on
+    128 x 256 tiles: every column of sampled rows, the seam between the two launches among them."""
+    rng = np.random.default_rng(M + N + K)
+    A = rng.normal(0, 1, (M, K)).astype(np.float32)
+    B = rng.normal(0, 0.02, (2 * N, K)).astype(np.float16)
+    rows = np.unique(np.concatenate([[0, 255, 256, M - 1], rng.integers(0, M, 24)]))
+    if amode == "f8":
+        dA, hi, val = f8_buffer(dev, A)
+        prod = T.f8lo_product(hi[rows], val[rows] - hi[rows].astype(np.float64), B)
+    else:
+        hi = A.astype(np.float16)
+        lo = (A - hi.astype(np.float32)).astype(np.float16)
+        dA = dev.put(np.concatenate([hi, lo]))
+        prod = (hi[rows].astype(np.float64) + lo[rows].astype(np.float64)) @ B.astype(np.float64).T
+    C = dev.put(np.zeros((2 * M, N), np.float16))
+    flags = 3 | vsl.GEMM_C_X2 | (vsl.GEMM_A_F8 if amode == "f8" else vsl.GEMM_A_X2)
+    ok(vsl, H.vsl_gemm_f16(dev.p(dA), dev.p(dev.put(B)), M, N, K, dev.p(C), flags, None))
+    o = dev.get(C).astype(np.float64)
+    ref = prod[:, :N] / (1.0 + np.exp(-prod[:, :N])) * prod[:, N:]
+    assert rel_err(o[rows] + o[M + rows], ref) < 2e-6
+
+
 @pytest.mark.parametrize("M,N,K,epi", [
     (512, 4096, 14336, 2),   # 8B down projection of a 512-row chunk
     (512, 6144, 4096, 0),    # 8B QKV (128 x 192 tiles)

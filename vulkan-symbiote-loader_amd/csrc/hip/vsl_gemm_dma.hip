@@ -107,6 +107,11 @@ struct B8Shift {
 };
 inline B8Shift b8_shift(int s) { return {std::ldexp(1.0f, -s), 127 - s}; }
 
+// Column tiles first .. first + n - 1 of the product (a launch may cover part of its width).
+struct ColTiles {
+    uint32_t first, n;
+};
+
 // SK (split K): the block's work item is (k chunk, tile); it multiplies K / ksplit of K and stores
 // the fp32 partial tile to ws[chunk][M][N]; k_splitk_reduce sums the chunks in order and applies the
 // epilogue (SwiGLU is not split).
@@ -120,7 +125,7 @@ inline B8Shift b8_shift(int s) { return {std::ldexp(1.0f, -s), 127 - s}; }
 template <class G, int EPI, int AM, int CM, bool SK>
 __global__ __launch_bounds__(G::NT) void k_gemm_dma(const vsl_half* __restrict__ A, const vsl_half* __restrict__ B,
                                                        uint32_t M, uint32_t N, uint32_t K, void* __restrict__ C,
-                                                       float* __restrict__ ws, uint32_t ksplit, B8Shift b8) {
+                                                       float* __restrict__ ws, uint32_t ksplit, B8Shift b8, ColTiles ct) {
     constexpr int BM = G::BM, BN = G::BN, BK = G::BK, WM = G::WM, WN = G::WN, FM = G::FM, FN = G::FN;
     constexpr int ACH = G::ACH, BCH = G::BCH, LCH = G::LCH, STAGE = G::STAGE, CPR = G::CPR, CPR8 = G::CPR8;
     constexpr int NBUF = G::NBUF, KS = G::KS;
@@ -139,7 +144,7 @@ __global__ __launch_bounds__(G::NT) void k_gemm_dma(const vsl_half* __restrict__
     const int wm = wave / WGN, wn = wave % WGN;
     static_assert(!SK || EPI != VSL_EPI_SWIGLU, "SwiGLU is not split over K");
     const uint32_t ncols = EPI == VSL_EPI_SWIGLU ? BN / 2 : BN;
-    const uint32_t n_m = (M + BM - 1) / BM, n_tiles = n_m * (N / ncols);
+    const uint32_t n_m = (M + BM - 1) / BM, n_tiles = n_m * ct.n;
     const uint32_t n_items = SK ? n_tiles * ksplit : n_tiles;
     // XCD-aware tile order: workgroups go to the 8 XCDs round-robin by block id; each XCD takes a
     // contiguous range of work items, m fastest, so blocks sharing a B tile share an L2
@@ -148,7 +153,7 @@ __global__ __launch_bounds__(G::NT) void k_gemm_dma(const vsl_half* __restrict__
     if (slot >= per || item >= n_items) return;
     const uint32_t kc = SK ? item / n_tiles : 0, t = SK ? item % n_tiles : item;
     const uint32_t mt = t % n_m, nt = t / n_m;
-    const uint32_t m0 = mt * BM, nout0 = nt * ncols;
+    const uint32_t m0 = mt * BM, nout0 = (ct.first + nt) * ncols;
     const uint32_t kspan = SK ? K / ksplit : K;  // K range of this block: [kc * kspan, (kc + 1) * kspan)
     const size_t plane = (size_t)M * K;
     // the fp8 lo plane follows the hi plane (bytes)
@@ -515,28 +520,28 @@ uint32_t dma_tiles(uint32_t M, uint32_t N) {
 }
 
 template <class G, int EPI, int AM>
-void launch_cm(uint32_t blocks, hipStream_t s, const vsl_half* a, const vsl_half* b, uint32_t M, uint32_t N,
+void launch_cm(ColTiles ct, hipStream_t s, const vsl_half* a, const vsl_half* b, uint32_t M, uint32_t N,
                uint32_t K, void* C, int cm, B8Shift b8) {
+    const uint32_t blocks = ((M + G::BM - 1) / G::BM * ct.n + 7) / 8 * 8;  // whole XCD ranges
     if constexpr (EPI == VSL_EPI_SWIGLU) {
         if (cm == kCX2) {
-            k_gemm_dma<G, EPI, AM, kCX2, false><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8);
+            k_gemm_dma<G, EPI, AM, kCX2, false><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8, ct);
             return;
         }
         if (cm == kCF8) {
-            k_gemm_dma<G, EPI, AM, kCF8, false><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8);
+            k_gemm_dma<G, EPI, AM, kCF8, false><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8, ct);
             return;
         }
     }
-    k_gemm_dma<G, EPI, AM, kC1, false><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8);
+    k_gemm_dma<G, EPI, AM, kC1, false><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8, ct);
 }
 
 template <class P, int EPI>
-void launch_cfg(uint32_t tiles, hipStream_t s, const vsl_half* a, const vsl_half* b, uint32_t M, uint32_t N,
+void launch_cfg(ColTiles ct, hipStream_t s, const vsl_half* a, const vsl_half* b, uint32_t M, uint32_t N,
                 uint32_t K, void* C, int am, int cm, B8Shift b8) {
-    const uint32_t blocks = ((tiles + 7) / 8) * 8;  // whole XCD ranges
-    if (am == kAX2) launch_cm<typename P::Two, EPI, kAX2>(blocks, s, a, b, M, N, K, C, cm, b8);
-    else if (am == kAF8) launch_cm<typename P::F8, EPI, kAF8>(blocks, s, a, b, M, N, K, C, cm, b8);
-    else launch_cm<typename P::One, EPI, kA1>(blocks, s, a, b, M, N, K, C, cm, b8);
+    if (am == kAX2) launch_cm<typename P::Two, EPI, kAX2>(ct, s, a, b, M, N, K, C, cm, b8);
+    else if (am == kAF8) launch_cm<typename P::F8, EPI, kAF8>(ct, s, a, b, M, N, K, C, cm, b8);
+    else launch_cm<typename P::One, EPI, kA1>(ct, s, a, b, M, N, K, C, cm, b8);
 }
 
 // split-K GEMM (partials, the epilogue's type only selects the reduce kernel)
@@ -544,32 +549,49 @@ template <class P>
 void launch_splitk(uint32_t items, hipStream_t s, const vsl_half* a, const vsl_half* b, uint32_t M, uint32_t N,
                    uint32_t K, float* ws, uint32_t ksplit, int am, B8Shift b8) {
     const uint32_t blocks = ((items + 7) / 8) * 8;
+    const ColTiles ct{0, N / (uint32_t)P::One::BN};
     if (am == kAX2)
         k_gemm_dma<typename P::Two, VSL_EPI_STORE_F32, kAX2, kC1, true><<<blocks, P::Two::NT, 0, s>>>(
-            a, b, M, N, K, nullptr, ws, ksplit, b8);
+            a, b, M, N, K, nullptr, ws, ksplit, b8, ct);
     else if (am == kAF8)
         k_gemm_dma<typename P::F8, VSL_EPI_STORE_F32, kAF8, kC1, true><<<blocks, P::F8::NT, 0, s>>>(
-            a, b, M, N, K, nullptr, ws, ksplit, b8);
+            a, b, M, N, K, nullptr, ws, ksplit, b8, ct);
     else
         k_gemm_dma<typename P::One, VSL_EPI_STORE_F32, kA1, kC1, true><<<blocks, P::One::NT, 0, s>>>(
-            a, b, M, N, K, nullptr, ws, ksplit, b8);
+            a, b, M, N, K, nullptr, ws, ksplit, b8, ct);
+}
+
+// Whole rounds of 256 x 256 tiles, the rest of the columns on 128 x 256 tiles: the columns for the first,
+// or all of them where that costs no less. A 128 x 256 tile takes ~0.6 of a 256 x 256 one (fp8-lo, K =
+// 4096: 108 against 180 us a round of 256), so a last round less than half full is halved instead of
+// left idle: the layer's prompt pass of 8B at 2048 rows (896 gate/up tiles, 3.5 rounds) 1950 -> 1915 us, 700
+// rows (336 tiles) 689 -> 643, 1200 rows 1092 -> 1044. (One-plane A, whose ratio differs, keeps whole tiles.)
+template <int EPI>
+uint32_t big_columns(uint32_t M, uint32_t N) {
+    constexpr uint32_t kCUs = 256;
+    const uint32_t cols = N / (EPI == VSL_EPI_SWIGLU ? 128 : 256), n_m = (M + 255) / 256, n_m2 = (M + 127) / 128;
+    const uint32_t tiles = n_m * cols, full = tiles / kCUs;
+    if (!full || tiles % kCUs == 0) return cols;
+    const uint32_t big = full * kCUs / n_m;
+    const uint32_t rest = ((cols - big) * n_m2 + kCUs - 1) / kCUs;
+    return big && 0.6 * rest < 0.9 ? big : cols;
 }
 
 template <int EPI>
 int launch_epi(int cfg, hipStream_t s, const vsl_half* a, const vsl_half* b, uint32_t M, uint32_t N, uint32_t K,
                void* C, int am, int cm, B8Shift b8) {
+    const uint32_t per = EPI == VSL_EPI_SWIGLU ? 2 : 1;  // output columns are half a tile's B rows
     if (cfg == 0) {
-        const uint32_t t = dma_tiles<DmaBig::One, EPI>(M, N);
-        if (!t) return -1;
-        launch_cfg<DmaBig, EPI>(t, s, a, b, M, N, K, C, am, cm, b8);
+        if (!dma_tiles<DmaBig::One, EPI>(M, N)) return -1;
+        const uint32_t cols = N * per / 256, big = am == kA1 ? cols : big_columns<EPI>(M, N);
+        launch_cfg<DmaBig, EPI>({0, big}, s, a, b, M, N, K, C, am, cm, b8);
+        if (big < cols) launch_cfg<DmaMid, EPI>({big, cols - big}, s, a, b, M, N, K, C, am, cm, b8);
     } else if (cfg == 1) {
-        const uint32_t t = dma_tiles<DmaMid::One, EPI>(M, N);
-        if (!t) return -1;
-        launch_cfg<DmaMid, EPI>(t, s, a, b, M, N, K, C, am, cm, b8);
+        if (!dma_tiles<DmaMid::One, EPI>(M, N)) return -1;
+        launch_cfg<DmaMid, EPI>({0, N * per / 256}, s, a, b, M, N, K, C, am, cm, b8);
     } else {
-        const uint32_t t = dma_tiles<DmaSmall::One, EPI>(M, N);
-        if (!t) return -1;
-        launch_cfg<DmaSmall, EPI>(t, s, a, b, M, N, K, C, am, cm, b8);
+        if (!dma_tiles<DmaSmall::One, EPI>(M, N)) return -1;
+        launch_cfg<DmaSmall, EPI>({0, N * per / 128}, s, a, b, M, N, K, C, am, cm, b8);
     }
     return 0;
 }
