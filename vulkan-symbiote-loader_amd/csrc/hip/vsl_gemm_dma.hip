@@ -624,6 +624,10 @@ uint32_t vsl_gemm_splitk_plan(uint32_t M, uint32_t N, uint32_t K, int epi, uint3
     const uint32_t tiles = dma_tiles<DmaMid::One, VSL_EPI_STORE_F32>(M, N);
     if (!tiles || ((uint64_t)M * K * 2) >> 32 || ((uint64_t)N * K * 2) >> 32) return 0;
     auto take = [&](uint32_t ks) {
+        // half the chunks where they take half the rounds of 256 blocks: as much multiplying per CU, half
+        // the partials (a layer's prompt pass: 1B 600 rows, O and down at 40 tiles and 8 -> 4 chunks, 236.7 ->
+        // 219.5 us; 1B 300 rows 147.2 -> 142.7; 8B 300 rows 370.1 -> 365.8)
+        while (ks > 2 && (tiles * ks + 255) / 256 >= 2 * ((tiles * ks / 2 + 255) / 256)) ks /= 2;
         if (ws_bytes) *ws_bytes = (uint64_t)ks * M * N * 4;
         return ks;
     };
