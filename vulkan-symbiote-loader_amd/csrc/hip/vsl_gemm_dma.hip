@@ -613,6 +613,16 @@ uint32_t vsl_gemm_dma_tiles(int cfg, uint32_t M, uint32_t N, uint32_t K, int epi
     return sw ? dma_tiles<DmaSmall::One, VSL_EPI_SWIGLU>(M, N) : dma_tiles<DmaSmall::One, VSL_EPI_STORE_F32>(M, N);
 }
 
+// Which tile takes the K-split partials: the 128 x 192 tile when its whole rounds of 256 work items
+// cost less than the 128 x 256 tile's (tile area x rounds), else 128 x 256.
+static bool splitk_narrow(uint32_t M, uint32_t N, uint32_t ksplit) {
+    const uint64_t tq = dma_tiles<DmaQ::One, VSL_EPI_STORE_F32>(M, N);
+    const uint64_t tm = dma_tiles<DmaMid::One, VSL_EPI_STORE_F32>(M, N);
+    if (!tq || !tm) return false;
+    const uint64_t rq = (tq * ksplit + 255) / 256, rm = (tm * ksplit + 255) / 256;
+    return rq * 192 < rm * 256;
+}
+
 // Split-K plan for shapes whose tiles leave CUs idle: the 128 x 256 tiling with the smallest split
 // in {2, 4, 8} that gives >= min_items work items and >= 512 of K per chunk; else (few rows, e.g. a
 // 128-token prompt) the smallest split up to 32 with >= 128 of K per chunk that reaches min_items, or
@@ -626,8 +636,13 @@ uint32_t vsl_gemm_splitk_plan(uint32_t M, uint32_t N, uint32_t K, int epi, uint3
     auto take = [&](uint32_t ks) {
         // half the chunks where they take half the rounds of 256 blocks: as much multiplying per CU, half
         // the partials (a layer's prompt pass: 1B 600 rows, O and down at 40 tiles and 8 -> 4 chunks, 236.7 ->
-        // 219.5 us; 1B 300 rows 147.2 -> 142.7; 8B 300 rows 370.1 -> 365.8)
-        while (ks > 2 && (tiles * ks + 255) / 256 >= 2 * ((tiles * ks / 2 + 255) / 256)) ks /= 2;
+        // 219.5 us; 1B 300 rows 147.2 -> 142.7; 8B 300 rows 370.1 -> 365.8); down to one chunk where its
+        // tiles still fill five eighths of the CUs (8B QKV of 700 rows 659 -> 645, of 850 rows 753 -> 741, O and
+        // down of 1400 rows, 176 tiles, 1286 -> 1254; of 1100 rows, 144 tiles, two chunks 1045 against 1053)
+        while (ks > 1 && (tiles * ks + 255) / 256 >= 2 * ((tiles * ks / 2 + 255) / 256)) {
+            if (ks == 2 && (splitk_narrow(M, N, 1) ? dma_tiles<DmaQ::One, VSL_EPI_STORE_F32>(M, N) : tiles) < 160) break;
+            ks /= 2;
+        }
         if (ws_bytes) *ws_bytes = (uint64_t)ks * M * N * 4;
         return ks;
     };
@@ -640,16 +655,6 @@ uint32_t vsl_gemm_splitk_plan(uint32_t M, uint32_t N, uint32_t K, int epi, uint3
         widest = ks;
     }
     return widest && tiles * widest >= 64 ? take(widest) : 0;
-}
-
-// Which tile takes the K-split partials: the 128 x 192 tile when its whole rounds of 256 work items
-// cost less than the 128 x 256 tile's (tile area x rounds), else 128 x 256.
-static bool splitk_narrow(uint32_t M, uint32_t N, uint32_t ksplit) {
-    const uint64_t tq = dma_tiles<DmaQ::One, VSL_EPI_STORE_F32>(M, N);
-    const uint64_t tm = dma_tiles<DmaMid::One, VSL_EPI_STORE_F32>(M, N);
-    if (!tq || !tm) return false;
-    const uint64_t rq = (tq * ksplit + 255) / 256, rm = (tm * ksplit + 255) / 256;
-    return rq * 192 < rm * 256;
 }
 
 void vsl_gemm_splitk_partials(uint32_t ksplit, void* stream, const void* A, const void* B, uint32_t M, uint32_t N,
