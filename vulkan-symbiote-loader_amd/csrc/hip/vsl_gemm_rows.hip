@@ -12,11 +12,15 @@
 // planes against 16 NF weight rows): loads of eight whole lines fetch them at 18 TB/s, loads in the
 // operand layout (64 bytes of each of 16 rows, adjacent lanes in different rows) at 8 TB/s.
 //
+// The weights of the wide blocks are loaded non-temporally, each line once (8B layer of 45 rows 140.6 -> 133.4
+// us, of 3 rows 117.0 -> 105.3); the narrow shapes' (NF = 1) are small and keep plain loads (45.0 against 47.1).
+//
 // A layer's prompt pass, before (the tiles of vsl_gemm_dma.hip) -> with this kernel, us: 8B 45 rows 170.3 ->
-// 142.8, 3 rows 158.6 -> 117.0, 64 rows 177.5 -> 161.2; 1B 45 rows 99.2 -> 76.3, 7 rows 89.3 -> 61.8; 70B 40
-// rows 624.6 -> 399.8; d 768 with 30 rows 88.6 -> 43.7. Also measured at 45 / 64 rows of the 8B layer: both
-// operands in the operand layout 156 / 181; the weights alone in it 144 / 171; two register sets ahead
-// instead of one 149 / 218 (the second set's copies and spills); eight waves of 32-column units 159 / 184.
+// 133.4, 3 rows 158.6 -> 105.3, 64 rows 177.5 -> 149.4; 1B 45 rows 99.2 -> 76.3, 7 rows 89.3 -> 61.8, 128 rows
+// 114.5 -> 102.0; 70B 40 rows 624.6 -> 357.0; d 768 with 30 rows 88.6 -> 45.0. Also measured at 45 / 64 rows of the 8B
+// layer, all with plain loads (this kernel 142.8 / 161.2): both operands in the operand layout 156 / 181; the
+// weights alone in it 144 / 171; two register sets ahead instead of one 149 / 218 (the second set's copies
+// and spills); eight waves of 32-column units 159 / 184.
 #include <hip/hip_runtime.h>
 
 #include "vsl_device.h"
@@ -116,7 +120,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void k_gemm_rows(const vsl_half* __r
             for (int j = 0; j < 2 * MT; ++j) u.lo[j] = load16<false>(Ak + (size_t)M * K + k0 + a_off[j]);
         }
 #pragma unroll
-        for (int j = 0; j < 2 * NF; ++j) u.b[j] = load16<false>(Bk + k0 + b_off[j]);
+        for (int j = 0; j < 2 * NF; ++j) u.b[j] = load16<(NF > 1)>(Bk + k0 + b_off[j]);
         __builtin_amdgcn_sched_barrier(0);
     };
     float4v acc[NF][MT];
