@@ -4,16 +4,19 @@
 // HBM-bound: W streams once, 2 B flops per 2 weight bytes against a ridge of ~300. On the matrix cores
 // (v_mfma_f32_16x16x32_f16, A = 16 rows of W) the operand of X is, per lane, eight consecutive k of one
 // column, which this layout scatters B elements apart: gathered from memory, eight 2-byte loads per
-// fragment for every one or two 16-byte loads of W, their issue bounds the kernel. Here a wave loads the 64 rows of X of
-// its unit as they lie (contiguous, 16 bytes per lane) together with its W fragments, one unit ahead,
-// and turns them in its own piece of LDS: no block barrier until the waves' sums meet. Block = 16 NF rows
-// of W; its WAVES waves take every WAVES-th 64-column unit of K (one 128-byte line of each row, its
-// halves in adjacent loads), and the 16 NF rows share each X unit: NF = 4 where that still gives three
-// quarters of the CUs a block, else 2 or 1 with as many more waves. The blocks of an XCD start at
-// different units, three apart: rows of a power-of-two stride put one unit of all rows on few memory
-// channels (14336 x 4096, B = 16: 26.1 us without, 22.8 with).
-// N x K, B (gathering kernel -> this one, us): 14336 x 4096, 16 30.5 -> 22.8; 4096 x 4096, 9 8.3 -> 7.4;
-// 1000 x 14336, 4 21.2 -> 17.5; 32000 x 2048, 16 35.2 -> 25.5.
+// fragment for every one or two 16-byte loads of W, their issue bounds the kernel. Here a wave loads the 64
+// rows of X of its unit as they lie (contiguous, 16 bytes per lane) and the weights by whole 128-byte lines
+// (eight lanes per row), one unit ahead, and turns both in its own piece of LDS: no block barrier until the
+// waves' sums meet. Block = 16 NF rows of W; its WAVES waves take every WAVES-th 64-column unit of K, and
+// the 16 NF rows share each X unit: NF = 4 where that still gives three quarters of the CUs a block, else 2
+// or 1 with as many more waves. The weights of the wide blocks are loaded non-temporally; those of one
+// fragment per block are small matrices (up to 6143 rows) that a repeated product finds in the cache. The
+// blocks of an XCD start at different units, three apart: rows of a power-of-two stride put one unit of
+// all rows on few memory channels.
+// N x K, B (gathering kernel -> this one, us): 14336 x 4096, 16 30.5 -> 18.9; 4096 x 4096, 9 8.3 -> 7.1;
+// 1000 x 14336, 4 21.2 -> 12.9; 32000 x 2048, 16 35.2 -> 22.1; 8000 x 8192, 12 37.8 -> 24.8. (Weights loaded in the
+// operand layout, 64 bytes of each of 16 rows: 22.4, 7.3, 17.3, 25.3, 27.9; non-temporal for all: 19.0, 8.1, 15.1,
+// 22.1, 24.1; every block starting at the same unit: 26.1 in the operand layout for the first shape.)
 #include <hip/hip_runtime.h>
 
 #include "vsl_device.h"
@@ -28,18 +31,20 @@ template <int NF, int WAVES, typename YT>
 __global__ __launch_bounds__(WAVES * 64) void k_skinny_rows(const vsl_half* __restrict__ W, uint32_t N, uint32_t K,
                                                             const vsl_half* __restrict__ X, uint32_t B, YT* __restrict__ Y) {
     constexpr uint32_t ROWS = 16 * NF;
-    __shared__ __attribute__((aligned(16))) vsl_half xs[WAVES][kUnit * 16];
+    // a wave's unit: the rows of X as they lie, then the weight rows (chunk c of row r at position
+    // c ^ ((r >> 1) & 7), so that the 16 rows of a fragment read fall in distinct banks)
+    __shared__ __attribute__((aligned(16))) vsl_half xs[WAVES][kUnit * 16 * (1 + NF)];
     __shared__ float part[WAVES][ROWS][17];
     const uint32_t lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t units = K / kUnit, nu = wave < units ? (units - 1 - wave) / WAVES + 1 : 0;
     const uint32_t rot = (blockIdx.x >> 3) * 3 % units;
     const uint32_t col = r16 < B ? r16 : B - 1;  // columns past B are not stored
-    const vsl_half* wrow[NF];
+    const vsl_half* wrow[2 * NF];  // load j: eight rows' whole lines, eight lanes per row
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-        const uint32_t row = blockIdx.x * ROWS + 16 * f + r16;  // rows past N re-read row N - 1, not stored
-        wrow[f] = W + (size_t)(row < N ? row : N - 1) * K + 8 * g;
+    for (int j = 0; j < 2 * NF; ++j) {
+        const uint32_t r = 8 * j + (lane >> 3), row = blockIdx.x * ROWS + r;  // rows past N re-read row N - 1, not stored
+        wrow[j] = W + (size_t)(row < N ? row : N - 1) * K + 8 * ((lane & 7) ^ ((r >> 1) & 7));
     }
     const uint32_t chunks = 8 * B;  // 16-byte chunks of a unit of X (64 B halfs)
     uint32_t xc[2];
@@ -47,8 +52,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_skinny_rows(const vsl_half* __re
     for (int j = 0; j < 2; ++j) xc[j] = 8 * (lane + 64 * j < chunks ? lane + 64 * j : chunks - 1);
 
     struct Unit {
-        half8 w[2][NF];
-        uint4 x[2];
+        uint4 w[2 * NF], x[2];
     };
     auto load = [&](Unit& u, uint32_t i) {
         uint32_t un = wave + i * WAVES + rot;
@@ -57,9 +61,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_skinny_rows(const vsl_half* __re
 #pragma unroll
         for (int j = 0; j < 2; ++j) u.x[j] = load16<false>(X + (size_t)k0 * B + xc[j]);
 #pragma unroll
-        for (int f = 0; f < NF; ++f)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) u.w[t][f] = *reinterpret_cast<const half8*>(wrow[f] + k0 + 32 * t);
+        for (int j = 0; j < 2 * NF; ++j) u.w[j] = load16<(NF > 1)>(wrow[j] + k0);
         __builtin_amdgcn_sched_barrier(0);
     };
     float4v acc[NF];
@@ -74,6 +76,9 @@ __global__ __launch_bounds__(WAVES * 64) void k_skinny_rows(const vsl_half* __re
     auto compute = [&](const Unit& u) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) *reinterpret_cast<uint4*>(&xs[wave][xc[j]]) = u.x[j];
+        vsl_half* const ws = &xs[wave][kUnit * 16];
+#pragma unroll
+        for (int j = 0; j < 2 * NF; ++j) *reinterpret_cast<uint4*>(ws + j * 512 + lane * 8) = u.w[j];
         lds_order();
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -81,7 +86,10 @@ __global__ __launch_bounds__(WAVES * 64) void k_skinny_rows(const vsl_half* __re
 #pragma unroll
             for (int i = 0; i < 8; ++i) x[i] = xs[wave][(32 * t + 8 * g + i) * B + col];
 #pragma unroll
-            for (int f = 0; f < NF; ++f) acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(u.w[t][f], x, acc[f], 0, 0, 0);
+            for (int f = 0; f < NF; ++f) {
+                const half8 w = *reinterpret_cast<const half8*>(ws + f * 1024 + r16 * kUnit + ((4 * t + g) ^ (r16 >> 1)) * 8);
+                acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, acc[f], 0, 0, 0);
+            }
         }
         lds_order();
         __builtin_amdgcn_sched_barrier(0);
