@@ -733,6 +733,43 @@ def test_lm_head_samplers_match_general_path(vsl, orc, dev, H, name):
             assert np.array_equal(dev.get(logits), l, equal_nan=True)
 
 
+@pytest.mark.parametrize("V,T", [(20000, 1.0), (128256, 1.0), (300000, 1.0), (9000, 0.7)])
+def test_lm_head_reference_near_ties(vsl, dev, H, V, T):
+    """Reference mode picks the first index of the largest exp(l / T - max) / sum.  Two logits one ulp
+    apart below 1 have exponentials one ulp apart, and whether their quotients round to the same
+    probability turns on the last bits of the sum: the output stage and vsl_sample_logits, which add it
+    over different launches, name the same token for each of 32 such vectors (past 262144 logits the sums
+    take a second pass)."""
+    nb = H.vsl_lm_head_ws_blocks()
+    ws_v, ws_i = dev.empty((nb,), np.float32), dev.empty((nb,), np.int32)
+    out, toks, logits = dev.empty((1,), np.int32), dev.empty((1,), np.int32), dev.empty((V,), np.float32)
+    d = 8
+    x = np.zeros(d, np.float32)
+    x[0] = 1.0
+    E = dev.put(np.zeros((V, d), np.float32))
+    smp = vsl.Sampler(1, T, 1, 0, 9)
+    lower, got, want = [], [], []
+    for seed in range(32):
+        rng = np.random.default_rng([V, seed])
+        l = rng.normal(-3, 0.5, V).astype(np.float32)
+        a, b = np.sort(rng.choice(V, 2, replace=False))
+        l[b] = rng.uniform(0.5, 0.99) * T
+        l[a] = np.nextafter(l[b], np.float32(0))
+        W = np.zeros((V, d), np.float32)
+        W[:, 0] = l
+        dW, dl, dx = dev.put(W), dev.put(l), dev.put(x)
+        c = ctrl_buf(vsl, dev, H, 3, max_steps=4, cap=64)
+        ok(vsl, H.vsl_lm_head_sample(None, 1e-5, dev.p(dW), 0, V, d, dev.p(dx), dev.p(E), 0, dev.p(logits), smp,
+                                     dev.p(ws_v), dev.p(ws_i), dev.p(toks), dev.p(c), None))
+        ok(vsl, H.vsl_sample_logits(dev.p(dl), V, smp, 0, dev.p(out), None))
+        lower.append(int(a))
+        got.append(int(dev.get(toks)[0]))
+        want.append(int(dev.get(out)[0]))
+    assert got == want
+    if T == 1.0:  # both outcomes occur: the lower index where the quotients round together, else the larger logit
+        assert 0 < sum(t == a for t, a in zip(want, lower)) < 32
+
+
 def test_embed_clamps_out_of_range_ids(vsl, dev, H):
     """embedding_lookup.comp:32: an id at or past the vocabulary reads row V - 1 (fp16 and fp32 tables)."""
     V, d = 300, 64

@@ -1809,8 +1809,8 @@ __device__ __forceinline__ uint32_t block_sample(const float* __restrict__ logit
 // k = 3: 356.9 -> 325.5.
 struct LmBlocks {
     const float* val;     // per-block maxima; NaN logits never win, a block of NaNs alone holds -inf
-    const float* part;    // reference mode: per-block sums of exp (k_reference_sum)
-    uint32_t nb, n_part;  // nb <= kSampBlock blocks, n_part sums
+    const float* part;    // reference mode: kSampBlock sums of exp (k_reference_sum)
+    uint32_t nb;          // blocks, at most kSampBlock
     uint32_t rpb_log2;    // log2(rpb)
 };
 constexpr uint32_t kBlockTopK = 128;  // seeded top-k through the block maxima up to this k
@@ -1958,37 +1958,53 @@ __device__ bool topk_sample_blocks(const float* __restrict__ logits, uint32_t V,
     return true;
 }
 
-// Reference mode, first launch: sums of exp(l / T - max) over slices of the logits, one per block (one
-// block over V = 128256 logits is bound by its expf arithmetic and its misses; 256 blocks share them).
-// The maximum of l / T is that of the block maxima divided by T: a division by T > 0 keeps order.
-constexpr uint32_t kRefBlocks = 256;
-constexpr int kRefThreads = 256;
-static_assert(kRefBlocks <= kMaxLmBlocks, "the sums take the place of the block indices");
+// Reference mode, first launch: part[t], the sum of exp(l / T - max) that thread t of block_sample makes of
+// logits t, t + kSampBlock, ..., added in that order, so that the output stage and vsl_sample_logits divide
+// by the same sum and name the same token where probabilities nearly tie. A block makes kRefLanes of the
+// sums: its threads take the exponentials (a single block over V = 128256 logits is bound by their
+// arithmetic and its misses) and kRefLanes of them add those from LDS. The maximum of l / T is that of the
+// block maxima divided by T: a division by T > 0 keeps order.
+constexpr uint32_t kRefLanes = 16, kRefBlocks = kSampBlock / kRefLanes;
+constexpr int kRefThreads = 1024;
+constexpr uint32_t kRefRows = kRefThreads / kRefLanes;  // logits of each sum per pass over the block
+constexpr uint32_t kRefPasses = 4;
+static_assert((uint32_t)kSampBlock <= kMaxLmBlocks, "the sums take the place of the block indices");
 __device__ __forceinline__ float ref_scaled(float l, float temperature) { return temperature != 1.0f ? l / temperature : l; }
 
 __global__ __launch_bounds__(kRefThreads) void k_reference_sum(const float* __restrict__ logits, uint32_t V, float T,
                                                                const float* __restrict__ ws_val, uint32_t nb,
                                                                float* __restrict__ part, const vsl_ctrl* ctrl) {
     __shared__ float red[kRefThreads / 64];
+    __shared__ float s_e[kRefPasses * kRefRows][kRefLanes];
     if (ctrl->done) return;
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = threadIdx.x, c = tid % kRefLanes, r = tid / kRefLanes;
     float mx = -INFINITY;
     for (uint32_t b = tid; b < nb; b += kRefThreads) mx = fmaxf(mx, ref_scaled(ws_val[b], T));
     mx = wave_max_dpp(mx);
     if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
     for (int w = 0; w < kRefThreads / 64; ++w) mx = fmaxf(mx, red[w]);
-    __syncthreads();
+    const uint32_t rows = (V + kSampBlock - 1) / kSampBlock, t = blockIdx.x * kRefLanes + c;
     float sum = 0.f;
-    for (uint32_t i = blockIdx.x * kRefThreads + tid; i < V; i += kRefBlocks * kRefThreads)
-        sum += expf(ref_scaled(logits[i], T) - mx);
-    sum = wave_sum_dpp(sum);
-    if ((tid & 63) == 0) red[tid >> 6] = sum;
-    __syncthreads();
-    if (tid == 0) {
-        for (int w = 1; w < kRefThreads / 64; ++w) sum += red[w];
-        part[blockIdx.x] = sum;
+    for (uint32_t r0 = 0; r0 < rows; r0 += kRefPasses * kRefRows) {
+        const uint32_t left = rows - r0, n = left < kRefPasses * kRefRows ? left : kRefPasses * kRefRows;
+        float l[kRefPasses];
+#pragma unroll
+        for (uint32_t p = 0; p < kRefPasses; ++p) {
+            const uint64_t i = (uint64_t)(r0 + p * kRefRows + r) * kSampBlock + t;
+            l[p] = i < V ? logits[i] : -INFINITY;
+        }
+#pragma unroll
+        for (uint32_t p = 0; p < kRefPasses; ++p) {
+            const uint64_t i = (uint64_t)(r0 + p * kRefRows + r) * kSampBlock + t;
+            if (p * kRefRows + r < n) s_e[p * kRefRows + r][c] = i < V ? expf(ref_scaled(l[p], T) - mx) : 0.f;
+        }
+        __syncthreads();
+        if (r == 0)
+            for (uint32_t i = 0; i < n; ++i) sum += s_e[i][c];
+        __syncthreads();
     }
+    if (r == 0) part[t] = sum;
 }
 
 // Reference mode, second launch (see block_sample): the first index of the largest exp(l / T - max) /
@@ -2010,8 +2026,8 @@ __device__ uint32_t reference_sample_blocks(const float* __restrict__ logits, ui
     mx = s_f[0];
     for (int w = 1; w < kSampBlock / 64; ++w) mx = fmaxf(mx, s_f[w]);
     __syncthreads();
-    float sum = tid < lb.n_part ? lb.part[tid] : 0.f;
-    sum = wave_sum_dpp(sum);
+    float sum = lb.part[tid];  // the threads' sums, added as in block_sample
+    for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, VSL_WAVE);
     if (lane == 0) s_f[wave] = sum;
     if (bv - mx >= -kRefNear) s_blk[atomicAdd(&s_nblk, 1u)] = (uint16_t)tid;  // nb > 0: none only with a NaN sum
     __syncthreads();
@@ -3019,7 +3035,7 @@ extern "C" int vsl_lm_head_sample(const float* gamma, float eps, const void* W, 
     // the sampling kernel reads the block maxima first and then the blocks that matter
     const uint64_t key = vsl_derive_key(sampler.seed, "sampler");
     float* part = reinterpret_cast<float*>(ws_idx);
-    LmBlocks lb{ws_val, part, nb, kRefBlocks, 0};
+    LmBlocks lb{ws_val, part, nb, 0};
     while ((1u << lb.rpb_log2) < 2 * gemv_waves_k(d)) ++lb.rpb_log2;  // two rows per wave
     if (sampler.mode == VSL_SAMPLE_REFERENCE) {
         k_reference_sum<<<kRefBlocks, kRefThreads, 0, s>>>(logits, V, sampler.temperature, ws_val, nb, part, ctrl);
