@@ -288,7 +288,9 @@ int vsl_norm_swiglu(const float* x, const float* gamma, float eps, const void* W
  *   f = RMSNorm(x, gamma) (gamma may be NULL: no final norm); logits = W f (fp32 [V]);
  *   greedy: per-block argmax fused into the GEMV, reduced by a second launch;
  *   reference and top-k modes (T > 0): the GEMV writes logits and its per-block maxima, and a
- *   sampling launch (reference mode: two) reads the blocks that the maxima leave in question
+ *   sampling launch (reference mode: two) reads the blocks that the maxima leave in question; where
+ *   those are most of a small vocabulary, one launch streams the logits; the token is that of
+ *   vsl_sample_logits either way
  *   (top-k limit: min(top_k, V) <= VSL_MAX_TOP_K; otherwise VSL_E_UNSUPPORTED before any launch).
  *   The sampled token is written to tokens[ctrl->step]; then x <- embed[token] (the next step's
  *   embedding_lookup), ctrl->pos += 1, ctrl->step += 1, and done is set on max_steps / EOS.

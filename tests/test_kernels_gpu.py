@@ -733,13 +733,40 @@ def test_lm_head_samplers_match_general_path(vsl, orc, dev, H, name):
             assert np.array_equal(dev.get(logits), l, equal_nan=True)
 
 
+@pytest.mark.parametrize("V,mode,k", [
+    (8191, 1, 1), (8192, 1, 1),                      # reference: the last streaming size, the first through the maxima
+    (300, 2, 5), (300, 2, 6),                        # five groups of blocks: all of them bound the draw, or too few
+    (1536, 2, 24), (1530, 2, 24), (1600, 2, 25),     # as many groups as k; one row of blocks short; half as many again asked
+    (4096, 2, 43), (4096, 2, 44),                    # 64 groups, 64 and 66 asked
+    (2080, 2, 65), (2048, 2, 65), (4096, 2, 128), (4064, 2, 128),  # smaller groups past k = 64
+])
+def test_lm_head_sampler_routes(vsl, orc, dev, H, V, mode, k):
+    """Both sides of the line between sampling through the blocks' maxima and streaming the logits: the
+    oracle's token (reference mode: that of vsl_sample_logits too) and the logits, over four steps."""
+    rng = np.random.default_rng(V + k)
+    l = rng.normal(0, 1.3, V).astype(np.float32)
+    W, x = np.zeros((V, 8), np.float32), np.zeros(8, np.float32)
+    W[:, 0], x[0] = l, 1.0
+    nb = H.vsl_lm_head_ws_blocks()
+    ws_v, ws_i, out, toks = (dev.empty((n,), t) for n, t in ((nb, np.float32), (nb, np.int32), (1, np.int32), (4, np.int32)))
+    dW, dx, dl, logits = dev.put(W), dev.put(x), dev.put(l), dev.empty((V,), np.float32)
+    E = dev.put(np.broadcast_to(x, (V, 8)).copy())
+    smp, c = vsl.Sampler(mode, 0.8, k, 0, 9), ctrl_buf(vsl, dev, H, 3, max_steps=64, cap=64)
+    for step in range(4):
+        ok(vsl, H.vsl_lm_head_sample(None, 1e-5, dev.p(dW), 0, V, 8, dev.p(dx), dev.p(E), 0, dev.p(logits), smp,
+                                     dev.p(ws_v), dev.p(ws_i), dev.p(toks), dev.p(c), None))
+        ok(vsl, H.vsl_sample_logits(dev.p(dl), V, smp, step, dev.p(out), None))
+        assert int(dev.get(toks)[step]) == int(dev.get(out)[0]) == orc.sample(l, mode, 0.8, k, 9, step)
+    assert np.array_equal(dev.get(logits), l)
+
+
 @pytest.mark.parametrize("V,T", [(20000, 1.0), (128256, 1.0), (300000, 1.0), (9000, 0.7)])
 def test_lm_head_reference_near_ties(vsl, dev, H, V, T):
     """Reference mode picks the first index of the largest exp(l / T - max) / sum.  Two logits one ulp
     apart below 1 have exponentials one ulp apart, and whether their quotients round to the same
     probability turns on the last bits of the sum: the output stage and vsl_sample_logits, which add it
-    over different launches, name the same token for each of 32 such vectors (past 262144 logits the sums
-    take a second pass)."""
+    over different launches from 8192 logits on, name the same token for each of 32 such vectors (past 262144
+    logits the sums take a second pass)."""
     nb = H.vsl_lm_head_ws_blocks()
     ws_v, ws_i = dev.empty((nb,), np.float32), dev.empty((nb,), np.int32)
     out, toks, logits = dev.empty((1,), np.int32), dev.empty((1,), np.int32), dev.empty((V,), np.float32)

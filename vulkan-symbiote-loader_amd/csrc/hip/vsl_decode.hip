@@ -1851,6 +1851,7 @@ __device__ __forceinline__ void for_each_block_logit(const float* __restrict__ l
 // k, for ordinary logits) are ranked by counting, each of the 1024 threads comparing one of them
 // with a share of the others. Returns false, having drawn nothing, where the bound does not help: fewer
 // than k groups hold a number above -inf, or more than kSampBlock logits reach tau.
+__host__ __device__ constexpr uint32_t topk_groups(uint32_t k) { return k <= 64 ? 128u : 256u; }
 __device__ bool topk_sample_blocks(const float* __restrict__ logits, uint32_t V, const LmBlocks& lb, uint32_t k,
                                    float temperature, uint32_t k0, uint32_t k1, uint64_t step, uint64_t* s_cand,
                                    uint64_t* s_sort, uint32_t& tok) {
@@ -1860,7 +1861,7 @@ __device__ bool topk_sample_blocks(const float* __restrict__ logits, uint32_t V,
     __shared__ uint32_t s_nblk, s_n, s_tau32, s_out;
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t bkey = tid < lb.nb ? value_key(lb.val[tid]) : 0u;
-    const uint32_t ng = k <= 64 ? 128u : 256u;
+    const uint32_t ng = topk_groups(k);
     uint32_t gm = bkey;  // the group's maximum: four adjacent lanes, then the other four of the half row
     auto dpp_max = [](uint32_t v, uint32_t o) { return o > v ? o : v; };
     gm = dpp_max(gm, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)gm, 0xB1, 0xF, 0xF, false));
@@ -2057,21 +2058,27 @@ __global__ __launch_bounds__(kSampBlock) void k_sample_logits(const float* logit
     if (threadIdx.x == 0) *out = tok;
 }
 
-template <class ET>
+// MAXIMA: through the blocks' maxima (use_block_maxima); otherwise streaming the logits, in a kernel of its
+// own: carrying the other path costs it 1.5 us of instruction fetches and LDS.
+template <class ET, bool MAXIMA>
 __global__ __launch_bounds__(kSampBlock) void k_sample_finish(const float* logits, uint32_t V, uint32_t d, int mode,
                                                               float T, uint32_t top_k, uint32_t k0, uint32_t k1,
                                                               LmBlocks lb, const void* embed, float* x_next,
                                                               uint32_t* tokens, vsl_ctrl* ctrl) {
-    __shared__ uint64_t s_cand[kSampBlock];
-    __shared__ uint64_t s_sort[kSampBlock];
     if (ctrl->done) return;
     uint32_t tok;
-    if (mode == VSL_SAMPLE_REFERENCE) {
-        tok = reference_sample_blocks(logits, V, lb, T);
+    if constexpr (MAXIMA) {
+        __shared__ uint64_t s_cand[kSampBlock];
+        __shared__ uint64_t s_sort[kSampBlock];
+        if (mode == VSL_SAMPLE_REFERENCE) {
+            tok = reference_sample_blocks(logits, V, lb, T);
+        } else {
+            const uint32_t k = top_k > V ? V : top_k;
+            if (k > kBlockTopK || !topk_sample_blocks(logits, V, lb, k, T, k0, k1, ctrl->step, s_cand, s_sort, tok))
+                tok = block_sample(logits, V, mode, T, top_k, k0, k1, ctrl->step);
+        }
     } else {
-        const uint32_t k = top_k > V ? V : top_k;
-        if (k > kBlockTopK || !topk_sample_blocks(logits, V, lb, k, T, k0, k1, ctrl->step, s_cand, s_sort, tok))
-            tok = block_sample(logits, V, mode, T, top_k, k0, k1, ctrl->step);
+        tok = block_sample(logits, V, mode, T, top_k, k0, k1, ctrl->step);
     }
     finish_token<ET>(tok, V, d, embed, x_next, tokens, ctrl);
 }
@@ -3005,6 +3012,20 @@ static int check_sampler(const vsl_sampler& sp, uint32_t V, const char* who) {
     return VSL_OK;
 }
 
+// Whether the output stage samples through its nb blocks' maxima rather than by streaming the V logits
+// (the same token either way). Reference mode takes a launch more for it: output stage at V = 4096 14.6 us
+// streaming, 16.3 through the maxima, 7000 22.3 / 22.6, 8192 18.7 / 18.3, 32000 (K = 2048) 47.5 / 31.9. Top-k
+// needs k groups of blocks to bound the k-th logit, or the attempt is spent (V = 300, k = 6 16.0 / 19.6); up
+// to 64, where streaming is cheap, a bound that nearly all groups set also leaves many candidates: k = 44 of
+// 64 groups 18.5 / 18.3, 48 18.7 / 18.9, 64 20.1 / 24.9; k = 24 of 32 16.8 / 15.7, 32 16.9 / 17.8. Past 64
+// streaming takes a radix select (k = 65 of 65 groups 34.1 / 26.0, 128 of 128 40.2 / 32.9).
+static bool use_block_maxima(const vsl_sampler& sp, uint32_t V, uint32_t nb) {
+    if (sp.mode == VSL_SAMPLE_REFERENCE) return V >= 8192;
+    const uint32_t k = sp.top_k < V ? sp.top_k : V, per_group = kSampBlock / topk_groups(k);
+    const uint32_t groups = (nb + per_group - 1) / per_group;
+    return k <= kBlockTopK && groups >= (k > 24 && k <= 64 ? k + k / 2 : k);
+}
+
 extern "C" int vsl_lm_head_sample(const float* gamma, float eps, const void* W, int wdtype, uint32_t V, uint32_t d,
                                   float* x, const void* embed, int embed_dtype, float* logits, vsl_sampler sampler,
                                   float* ws_val, uint32_t* ws_idx, uint32_t* tokens, vsl_ctrl* ctrl, void* stream) {
@@ -3022,8 +3043,11 @@ extern "C" int vsl_lm_head_sample(const float* gamma, float eps, const void* W, 
     a.W = W; a.N = V; a.K = d; a.x = x; a.gamma = gamma; a.eps = eps; a.y = logits;
     a.ws_val = ws_val; a.ws_idx = ws_idx; a.tokens = tokens; a.embed = embed; a.x_next = x;
     a.ctrl = ctrl;
-    if (int rc = launch_gemv_w<2, EPI_ARGMAX>(wdtype, a, kMaxLmBlocks, s, "vsl_lm_head_sample")) return rc;
     const uint32_t nb = gemv_blocks_k<2, EPI_ARGMAX>(V, d, kMaxLmBlocks);
+    const bool maxima = fused || use_block_maxima(sampler, V, nb);
+    if (int rc = maxima ? launch_gemv_w<2, EPI_ARGMAX>(wdtype, a, kMaxLmBlocks, s, "vsl_lm_head_sample")
+                        : launch_gemv_w<2, EPI_STORE>(wdtype, a, 1u << 20, s, "vsl_lm_head_sample"))
+        return rc;
     if (fused) {
         if (embed_dtype == VSL_DT_F16)
             k_argmax_finish<WF16><<<1, kFinishThreads, 0, s>>>(ws_val, ws_idx, nb, V, d, embed, x, tokens, ctrl);
@@ -3032,21 +3056,20 @@ extern "C" int vsl_lm_head_sample(const float* gamma, float eps, const void* W, 
         HIP_TRY(hipGetLastError());
         return VSL_OK;
     }
-    // the sampling kernel reads the block maxima first and then the blocks that matter
     const uint64_t key = vsl_derive_key(sampler.seed, "sampler");
     float* part = reinterpret_cast<float*>(ws_idx);
     LmBlocks lb{ws_val, part, nb, 0};
     while ((1u << lb.rpb_log2) < 2 * gemv_waves_k(d)) ++lb.rpb_log2;  // two rows per wave
-    if (sampler.mode == VSL_SAMPLE_REFERENCE) {
+    if (sampler.mode == VSL_SAMPLE_REFERENCE && maxima) {
         k_reference_sum<<<kRefBlocks, kRefThreads, 0, s>>>(logits, V, sampler.temperature, ws_val, nb, part, ctrl);
         HIP_TRY(hipGetLastError());
     }
-    if (embed_dtype == VSL_DT_F16)
-        k_sample_finish<WF16><<<1, kSampBlock, 0, s>>>(logits, V, d, sampler.mode, sampler.temperature, sampler.top_k,
-                                                       (uint32_t)key, (uint32_t)(key >> 32), lb, embed, x, tokens, ctrl);
-    else
-        k_sample_finish<WF32><<<1, kSampBlock, 0, s>>>(logits, V, d, sampler.mode, sampler.temperature, sampler.top_k,
-                                                       (uint32_t)key, (uint32_t)(key >> 32), lb, embed, x, tokens, ctrl);
+    auto finish = [&](auto kernel) {
+        kernel<<<1, kSampBlock, 0, s>>>(logits, V, d, sampler.mode, sampler.temperature, sampler.top_k, (uint32_t)key,
+                                        (uint32_t)(key >> 32), lb, embed, x, tokens, ctrl);
+    };
+    if (embed_dtype == VSL_DT_F16) finish(maxima ? k_sample_finish<WF16, true> : k_sample_finish<WF16, false>);
+    else finish(maxima ? k_sample_finish<WF32, true> : k_sample_finish<WF32, false>);
     HIP_TRY(hipGetLastError());
     return VSL_OK;
 }
