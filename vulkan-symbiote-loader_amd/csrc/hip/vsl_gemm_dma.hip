@@ -107,7 +107,9 @@ struct B8Shift {
 };
 inline B8Shift b8_shift(int s) { return {std::ldexp(1.0f, -s), 127 - s}; }
 
-// Column tiles first .. first + n - 1 of the product (a launch may cover part of its width).
+// Column tiles first .. first + n - 1 of the product, for a launch that covers part of its width (PART).
+// Launches of the whole width (most calls) take their tile count from the shape: with the range in every
+// instance the 128 x 256 hi/lo SwiGLU tiles lost 2 % (8B gate/up of 256 rows 118.1 -> 120.3 us).
 struct ColTiles {
     uint32_t first, n;
 };
@@ -122,7 +124,7 @@ struct ColTiles {
 // and 2^-s, into the same accumulators. Operand slot j of lane group g in that MFMA is column 16 (j / 8) + 8 g + j % 8 of
 // the 64: the B fragment of k-step t supplies slots 8t..8t+7, and the lo plane's byte order
 // (lo8_pos) puts the A slots of a 32-column block in one 16-byte chunk per lane group.
-template <class G, int EPI, int AM, int CM, bool SK>
+template <class G, int EPI, int AM, int CM, bool SK, bool PART = false>
 __global__ __launch_bounds__(G::NT) void k_gemm_dma(const vsl_half* __restrict__ A, const vsl_half* __restrict__ B,
                                                        uint32_t M, uint32_t N, uint32_t K, void* __restrict__ C,
                                                        float* __restrict__ ws, uint32_t ksplit, B8Shift b8, ColTiles ct) {
@@ -144,7 +146,7 @@ __global__ __launch_bounds__(G::NT) void k_gemm_dma(const vsl_half* __restrict__
     const int wm = wave / WGN, wn = wave % WGN;
     static_assert(!SK || EPI != VSL_EPI_SWIGLU, "SwiGLU is not split over K");
     const uint32_t ncols = EPI == VSL_EPI_SWIGLU ? BN / 2 : BN;
-    const uint32_t n_m = (M + BM - 1) / BM, n_tiles = n_m * ct.n;
+    const uint32_t n_m = (M + BM - 1) / BM, n_tiles = n_m * (PART ? ct.n : N / ncols);
     const uint32_t n_items = SK ? n_tiles * ksplit : n_tiles;
     // XCD-aware tile order: workgroups go to the 8 XCDs round-robin by block id; each XCD takes a
     // contiguous range of work items, m fastest, so blocks sharing a B tile share an L2
@@ -153,7 +155,7 @@ __global__ __launch_bounds__(G::NT) void k_gemm_dma(const vsl_half* __restrict__
     if (slot >= per || item >= n_items) return;
     const uint32_t kc = SK ? item / n_tiles : 0, t = SK ? item % n_tiles : item;
     const uint32_t mt = t % n_m, nt = t / n_m;
-    const uint32_t m0 = mt * BM, nout0 = (ct.first + nt) * ncols;
+    const uint32_t m0 = mt * BM, nout0 = (PART ? ct.first + nt : nt) * ncols;
     const uint32_t kspan = SK ? K / ksplit : K;  // K range of this block: [kc * kspan, (kc + 1) * kspan)
     const size_t plane = (size_t)M * K;
     // the fp8 lo plane follows the hi plane (bytes)
@@ -519,21 +521,27 @@ uint32_t dma_tiles(uint32_t M, uint32_t N) {
     return N % ncols ? 0u : ((M + G::BM - 1) / G::BM) * (N / ncols);
 }
 
+template <class G, int EPI, int AM, int CM>
+void launch_part(ColTiles ct, hipStream_t s, const vsl_half* a, const vsl_half* b, uint32_t M, uint32_t N,
+                 uint32_t K, void* C, B8Shift b8) {
+    const uint32_t blocks = ((M + G::BM - 1) / G::BM * ct.n + 7) / 8 * 8;  // whole XCD ranges
+    const bool part = ct.n != N / (EPI == VSL_EPI_SWIGLU ? G::BN / 2 : G::BN);
+    if constexpr (AM != kA1 && G::BN == 256)  // the tiles that mixed rounds use
+        if (part) {
+            k_gemm_dma<G, EPI, AM, CM, false, true><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8, ct);
+            return;
+        }
+    k_gemm_dma<G, EPI, AM, CM, false><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8, ct);
+}
+
 template <class G, int EPI, int AM>
 void launch_cm(ColTiles ct, hipStream_t s, const vsl_half* a, const vsl_half* b, uint32_t M, uint32_t N,
                uint32_t K, void* C, int cm, B8Shift b8) {
-    const uint32_t blocks = ((M + G::BM - 1) / G::BM * ct.n + 7) / 8 * 8;  // whole XCD ranges
     if constexpr (EPI == VSL_EPI_SWIGLU) {
-        if (cm == kCX2) {
-            k_gemm_dma<G, EPI, AM, kCX2, false><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8, ct);
-            return;
-        }
-        if (cm == kCF8) {
-            k_gemm_dma<G, EPI, AM, kCF8, false><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8, ct);
-            return;
-        }
+        if (cm == kCX2) return launch_part<G, EPI, AM, kCX2>(ct, s, a, b, M, N, K, C, b8);
+        if (cm == kCF8) return launch_part<G, EPI, AM, kCF8>(ct, s, a, b, M, N, K, C, b8);
     }
-    k_gemm_dma<G, EPI, AM, kC1, false><<<blocks, G::NT, 0, s>>>(a, b, M, N, K, C, nullptr, 1, b8, ct);
+    launch_part<G, EPI, AM, kC1>(ct, s, a, b, M, N, K, C, b8);
 }
 
 template <class P, int EPI>
@@ -549,16 +557,15 @@ template <class P>
 void launch_splitk(uint32_t items, hipStream_t s, const vsl_half* a, const vsl_half* b, uint32_t M, uint32_t N,
                    uint32_t K, float* ws, uint32_t ksplit, int am, B8Shift b8) {
     const uint32_t blocks = ((items + 7) / 8) * 8;
-    const ColTiles ct{0, N / (uint32_t)P::One::BN};
     if (am == kAX2)
         k_gemm_dma<typename P::Two, VSL_EPI_STORE_F32, kAX2, kC1, true><<<blocks, P::Two::NT, 0, s>>>(
-            a, b, M, N, K, nullptr, ws, ksplit, b8, ct);
+            a, b, M, N, K, nullptr, ws, ksplit, b8, {});
     else if (am == kAF8)
         k_gemm_dma<typename P::F8, VSL_EPI_STORE_F32, kAF8, kC1, true><<<blocks, P::F8::NT, 0, s>>>(
-            a, b, M, N, K, nullptr, ws, ksplit, b8, ct);
+            a, b, M, N, K, nullptr, ws, ksplit, b8, {});
     else
         k_gemm_dma<typename P::One, VSL_EPI_STORE_F32, kA1, kC1, true><<<blocks, P::One::NT, 0, s>>>(
-            a, b, M, N, K, nullptr, ws, ksplit, b8, ct);
+            a, b, M, N, K, nullptr, ws, ksplit, b8, {});
 }
 
 // Whole rounds of 256 x 256 tiles, the rest of the columns on 128 x 256 tiles: the columns for the first,
