@@ -267,12 +267,15 @@ def test_gemm_f8lo_splitk(vsl, dev, H, M, N, K, epi):
     (20, 1984, 640, 3, "x2", "f16"),    # an odd multiple of 64 outputs
     (97, 3072, 2048, 0, "x2", None),    # two row blocks: 1B QKV and down projection, ragged and whole
     (128, 2048, 8192, 2, "x2", None),
-    (65, 8192, 2048, 3, "x2", "x2"), (128, 8192, 2048, 3, "x2", "x2"),
+    (65, 5632, 512, 3, "x2", "x2"), (96, 6080, 256, 3, "x2", "f16"),     # SwiGLU on two row blocks
+    (97, 4096, 1024, 3, "x2", "x2"), (128, 2048, 768, 3, "x2", "x2"),
+    (97, 4160, 1024, 3, "x2", "x2"),                                     # and the general tiles: too many rows,
+    (65, 8192, 2048, 3, "x2", "x2"), (128, 8192, 2048, 3, "x2", "x2"),   # or wide enough for those of 64 x 128
     (30, 768, 2048, 2, "x2", None),     # too narrow for a K split: 16 weight rows per block
     (5, 1280, 768, 0, "x2", None), (100, 768, 768, 1, "x2", None), (64, 256, 256, 2, "f8", None),
 ])
 def test_gemm_few_rows(vsl, dev, H, M, N, K, epi, amode, cmode):
-    """Chunks of up to 128 rows on the few-row kernel: every row tile count, block width, chunk count and
+    """Chunks of up to 128 rows on the few-row kernel (and at the edges of its range): every row tile count, block width, chunk count and
     units-per-wave remainder, against the fp64 product of the carried activations with the fp16 weights
     (an F16F8 lo plane is widened exactly, so the weights are not rounded to e4m3 here)."""
     rng = np.random.default_rng(M + N + K + epi)

@@ -17,7 +17,7 @@
 //
 // A layer's prompt pass, before (the tiles of vsl_gemm_dma.hip) -> with this kernel, us: 8B 45 rows 170.3 ->
 // 133.4, 3 rows 158.6 -> 105.3, 64 rows 177.5 -> 149.4; 1B 45 rows 99.2 -> 76.3, 7 rows 89.3 -> 61.8, 128 rows
-// 114.5 -> 102.0; 70B 40 rows 624.6 -> 357.0; d 768 with 30 rows 88.6 -> 45.0. Also measured at 45 / 64 rows of the 8B
+// 108.1 -> 96.8; 70B 40 rows 624.6 -> 357.0; d 768 with 30 rows 88.6 -> 45.0. Also measured at 45 / 64 rows of the 8B
 // layer, all with plain loads (this kernel 142.8 / 161.2): both operands in the operand layout 156 / 181; the
 // weights alone in it 144 / 171; two register sets ahead instead of one 149 / 218 (the second set's copies
 // and spills); eight waves of 32-column units 159 / 184.
@@ -294,8 +294,8 @@ struct RowsPlan {
 // partials' traffic (written and read, 4 bytes) shared by all. One wide block per CU beats two narrow ones
 // (4 x 16 rows everywhere: 8B layer of 45 rows 143 -> 171-188 us, of 3 rows 117 -> 133). More than 64 rows
 // run as two row blocks that share their weights through L2, in one round of blocks and for the narrow
-// models' products only (N or K up to 2048: the 1B layer of 90 rows 107.6 -> 93.9 us, of 128 rows 114.5 ->
-// 104.5); past that the activations read by every block outweigh what the general tiles waste (8B layer
+// models' products only (N or K up to 2048: the 1B layer's QKV of 128 rows 22.4 -> 15.8 us, O 22.1 -> 15.6,
+// down 27.7 -> 25.5); past that the activations read by every block outweigh what the general tiles waste (8B layer
 // of 100 rows 206.9 -> 215.9 with them, and 236 where gate/up took two rounds).
 RowsPlan rows_plan(uint32_t M, uint32_t N, uint32_t K, bool sw, int am, uint32_t max_ks) {
     RowsPlan best;

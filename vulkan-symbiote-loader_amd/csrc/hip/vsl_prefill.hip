@@ -862,9 +862,15 @@ static int launch_gemm(hipStream_t s, const vsl_half* a, const vsl_half* b, uint
                        void* C, int am, int cm, float* ws, uint64_t ws_bytes, int b8s) {
     auto blocks = [](uint32_t tiles) { return ((tiles + 7) / 8) * 8; };  // whole XCD ranges (tile_of)
     // few rows of a split A: the SwiGLU product streams its weights once (the fp8 forms on the shapes that
-    // the direct-to-LDS tiles take)
+    // the direct-to-LDS tiles take). Past 64 rows it takes two row blocks, and the 64 x 128 direct-to-LDS
+    // tiles are faster where they cover the CUs: outputs x K, us, those tiles / two row blocks: 6144 x 2048 of
+    // 65 rows 21.9 / 24.4; 8192 x 2048 (1B) of 100 rows 25.9 / 30.1, of 128 rows 28.0 / 30.4 (weights from
+    // memory; resident ones 24.5 / 31.5, 24.9 / 31.4). Narrower, against the register-staged tiles: 4096 x 2048
+    // of 128 rows 27.1 / 19.9, 5632 x 2048 of 96 rows 27.9 / 23.9; more than 96 rows of more than 4096 outputs
+    // have too few blocks of too many rows: 5120 x 1024 of 128 rows 16.5 / 18.5, x 2048 27.8 / 28.1.
     if constexpr (EPI == VSL_EPI_SWIGLU) {
-        if (((am != kGemmAF8 && cm != kGemmCF8) || vsl_gemm_dma_tiles(1, M, N, K, EPI)) &&
+        const bool two_blocks = vsl_gemm_dma_tiles(2, M, N, K, EPI) < kDmaMinTiles && (M <= 96 || N <= 4096);
+        if ((M <= 64 || two_blocks) && ((am != kGemmAF8 && cm != kGemmCF8) || vsl_gemm_dma_tiles(1, M, N, K, EPI)) &&
             vsl_gemm_rows_direct(s, a, b, M, N, K, C, EPI, am, cm))
             return VSL_OK;
     }
