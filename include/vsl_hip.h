@@ -340,17 +340,19 @@ int vsl_gemm_f16(const void* A, const void* B, uint32_t M, uint32_t N, uint32_t 
                  void* stream);
 /* The same with an fp32 workspace (16-byte aligned): shapes whose output tiles would leave CUs idle
  * (e.g. M = 512 against N = 4096) are split over K, the partials summed in a fixed order by a second
- * launch that applies the epilogue (not for VSL_EPI_SWIGLU).  vsl_gemm_f16_ws_bytes gives the bytes a
- * shape uses (0: no split, the workspace is not touched); with less than that the call runs
- * unsplit. */
+ * launch that applies the epilogue (not for VSL_EPI_SWIGLU).  vsl_gemm_f16_ws_bytes gives the bytes
+ * within which the call splits (0: no split, the workspace is not touched; few-row calls use at most
+ * that); with less than that the call runs unsplit.  The plan depends on the form of A: the bytes are
+ * those of the form among the flags, and without one they are enough for every form. */
 int vsl_gemm_f16_ws(const void* A, const void* B, uint32_t M, uint32_t N, uint32_t K, void* C, int epilogue,
                     void* workspace, uint64_t ws_bytes, void* stream);
 uint64_t vsl_gemm_f16_ws_bytes(uint32_t M, uint32_t N, uint32_t K, int epilogue);
 /* 1 when vsl_gemm_f16_ws (with vsl_gemm_f16_ws_bytes of workspace) runs this shape on the
  * direct-to-LDS kernel -- the one with the F8 forms -- through whole tiles that cover three quarters
- * of the CUs (192 tiles of 256 x 256 or 128 x 256), or through a K split: the smallest split giving
- * 192 work items where K allows one, else the widest split K allows when that gives at least 64
- * items (few-row shapes such as a 128-row prompt against N = 2048); 0 when it would take the
+ * of the CUs (192 tiles of 256 x 256 or 128 x 256), or through a K split: one giving 192 work items
+ * where K allows it, halved (possibly to one chunk of fewer items) where that is faster, else the widest
+ * split K allows when that gives at least 64 items (few-row shapes such as a 128-row prompt against N =
+ * 2048; up to 128 rows of a split A such shapes run on the few-row kernel instead); 0 when it would take the
  * register-staged kernel instead (an F8 form then forces the direct-to-LDS tiles at lower occupancy,
  * e.g. a 128-row SwiGLU on 64 tiles). */
 int vsl_gemm_f16_direct(uint32_t M, uint32_t N, uint32_t K, int epilogue);

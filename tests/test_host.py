@@ -67,6 +67,36 @@ def test_gemm_direct_query(vsl):
     assert H.vsl_gemm_f16_direct(512, 4096, 4000, F32) == 0      # K not a multiple of 128
 
 
+def test_gemm_splitk_plan_by_form(vsl):
+    """The K split per form of A, read off vsl_gemm_f16_ws_bytes (chunks x M x N x 4, host arithmetic only):
+    halved where half the chunks measured faster for that form, and enough for every form without one."""
+    H = vsl.hip()
+    RES, X2, F8 = 2, vsl.GEMM_A_X2, vsl.GEMM_A_F8
+
+    def chunks(M, N, K, flags):
+        b = H.vsl_gemm_f16_ws_bytes(M, N, K, RES | flags)
+        assert b % (4 * M * N) == 0
+        return b // (4 * M * N)
+
+    for M, N, K, one, f8, x2 in [
+        (640, 2048, 2048, 4, 4, 4),      # 40 tiles: 8 -> 4 for all
+        (1400, 4096, 4096, 1, 1, 1),     # 176 tiles: one chunk for all
+        (1100, 4096, 4096, 2, 2, 2),     # 144 tiles: two
+        (1274, 4096, 14336, 2, 2, 1),    # 160 wide tiles of ten row tiles, long chunks
+        (634, 8192, 8192, 1, 1, 1),      # ... of five row tiles
+        (1146, 2048, 14336, 4, 4, 2),    # 72 wide tiles
+        (1530, 3072, 8192, 2, 1, 1),     # 192 narrow tiles
+        (1530, 3072, 2048, 1, 1, 1),
+        (762, 3072, 14336, 4, 2, 2), (378, 6144, 8192, 2, 2, 2),
+        (1914, 2304, 14336, 2, 2, 1),    # 15 row tiles of 12 narrow ones
+    ]:
+        assert (chunks(M, N, K, 0), chunks(M, N, K, F8), chunks(M, N, K, X2)) == (one, f8, x2), (M, N, K)
+    for N in (1536, 2048, 2304, 4096, 6144, 8192):
+        for K in (1536, 4096, 14336):
+            for M in (1, 64, 128, *range(129, 2049, 77)):
+                assert chunks(M, N, K, 0) >= chunks(M, N, K, F8) >= chunks(M, N, K, X2)
+
+
 def test_no_cpu_fallback_in_the_product(vsl):
     """The product libraries link HIP and nothing from the oracle."""
     for lib in (vsl.HIP_LIB, vsl.ENGINE_LIB):

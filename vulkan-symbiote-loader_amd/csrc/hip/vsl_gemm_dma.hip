@@ -630,26 +630,44 @@ static bool splitk_narrow(uint32_t M, uint32_t N, uint32_t ksplit) {
     return rq * 192 < rm * 256;
 }
 
-// Split-K plan for shapes whose tiles leave CUs idle: the 128 x 256 tiling with the smallest split
-// in {2, 4, 8} that gives >= min_items work items and >= 512 of K per chunk; else (few rows, e.g. a
-// 128-token prompt) the smallest split up to 32 with >= 128 of K per chunk that reaches min_items, or
-// failing that the largest such split when it gives at least 64 items. Chunks are whole 128-wide
-// stage groups. Returns the split (0: none) and the fp32 workspace bytes it needs.
-uint32_t vsl_gemm_splitk_plan(uint32_t M, uint32_t N, uint32_t K, int epi, uint32_t min_items, uint64_t* ws_bytes) {
+// Whether half of ks chunks is faster: as much multiplying per CU and half the partials where it takes half
+// the rounds of 256 blocks (product with its residual + RMSNorm or store, us: 1B O of 600 rows, 40 tiles, 8
+// -> 4 chunks 32.6 -> 26.8; 1B QKV of 700 rows 38.7 -> 30.6), down to one chunk where its tiles still fill five
+// eighths of the CUs (8B O of 1400 rows, 176 tiles, 131.3 -> 113.5; 1100 rows, 144 tiles, stay at two). The
+// hi/lo form gains over all shapes measured (N 1536 to 10240, K 1536 to 28672). The others, whose blocks are
+// shorter, lose with long chunks where
+// - the narrow one-plane tiles (80 KB of LDS) no longer run two to a CU: 3072 x 14336 of 1530 rows one chunk
+//   +17 %, of 762 rows two +8 %, 9216 x 4096 of 506 rows -3 %, 3072 x 2048 of 1530 rows -3 %;
+// - the wide tiles leave CUs idle that a second, nearly empty round would not: one-plane / fp8 lo 4096 x
+//   14336 of 1274 rows (160 tiles) +6 / +6 %, 2048 x 14336 of 1146 rows (2 x 72) +4 / +5 %; of five to eight
+//   row tiles (8192 x 8192 of 634 rows) -9 / -4 %, from 176 tiles (4096 x 14336 of 1402 rows) -5 / -4 %;
+// - 15 row tiles of 12 narrow ones: fp8 lo 2304 x 14336 of 1914 rows +8 %.
+static bool splitk_half(uint32_t M, uint32_t N, uint32_t K, int am, uint32_t tiles, uint32_t ks) {
+    const uint32_t half = ks / 2, n_m = (M + 127) / 128, chunk = K / half;
+    if ((tiles * ks + 255) / 256 < 2 * ((tiles * half + 255) / 256)) return false;
+    const bool narrow = splitk_narrow(M, N, half);
+    const uint32_t items = (narrow ? dma_tiles<DmaQ::One, VSL_EPI_STORE_F32>(M, N) : tiles) * half;
+    if (half == 1 && items < 160) return false;
+    if (am == kAX2) return true;
+    if (am == kA1 && narrow && chunk > (half > 1 && n_m <= 10 ? 4096u : 2048u)) return false;
+    return chunk < 4096 || (narrow ? items >= 192 || n_m <= 12 : items >= 176 || (items >= 160 && n_m <= 8));
+}
+
+// Split-K plan for shapes whose tiles leave CUs idle. First the split that fills them: the 128 x 256 tiling
+// with the smallest split in {2, 4, 8} that gives >= min_items work items and >= 512 of K per chunk; else
+// (few rows, e.g. a 128-token prompt) the smallest split up to 32 with >= 128 of K per chunk that reaches
+// min_items, or failing that the largest such split when it gives at least 64 items; chunks are whole
+// 128-wide stage groups. Then it is halved while splitk_half allows, possibly to one chunk and to fewer
+// than min_items. Returns the split (0: none) and the fp32 workspace bytes it needs. For one shape a
+// one-plane A takes at least as many chunks as F16F8, and that at least as many as F16X2.
+uint32_t vsl_gemm_splitk_plan(uint32_t M, uint32_t N, uint32_t K, int epi, int am, uint32_t min_items,
+                              uint64_t* ws_bytes) {
     if (ws_bytes) *ws_bytes = 0;
     if (epi == VSL_EPI_SWIGLU || N % 4) return 0;
     const uint32_t tiles = dma_tiles<DmaMid::One, VSL_EPI_STORE_F32>(M, N);
     if (!tiles || ((uint64_t)M * K * 2) >> 32 || ((uint64_t)N * K * 2) >> 32) return 0;
     auto take = [&](uint32_t ks) {
-        // half the chunks where they take half the rounds of 256 blocks: as much multiplying per CU, half
-        // the partials (a layer's prompt pass: 1B 600 rows, O and down at 40 tiles and 8 -> 4 chunks, 236.7 ->
-        // 219.5 us; 1B 300 rows 147.2 -> 142.7; 8B 300 rows 370.1 -> 365.8); down to one chunk where its
-        // tiles still fill five eighths of the CUs (8B QKV of 700 rows 659 -> 645, of 850 rows 753 -> 741, O and
-        // down of 1400 rows, 176 tiles, 1286 -> 1254; of 1100 rows, 144 tiles, two chunks 1045 against 1053)
-        while (ks > 1 && (tiles * ks + 255) / 256 >= 2 * ((tiles * ks / 2 + 255) / 256)) {
-            if (ks == 2 && (splitk_narrow(M, N, 1) ? dma_tiles<DmaQ::One, VSL_EPI_STORE_F32>(M, N) : tiles) < 160) break;
-            ks /= 2;
-        }
+        while (ks > 1 && splitk_half(M, N, K, am, tiles, ks)) ks /= 2;
         if (ws_bytes) *ws_bytes = (uint64_t)ks * M * N * 4;
         return ks;
     };

@@ -45,7 +45,8 @@ int vsl_gemm_dma_launch(int cfg, void* stream, const void* A, const void* B, uin
                         void* C, int epi, int am, int cm, int b8s);
 // Split-K plan of the direct-to-LDS GEMM (k chunks of the 128 x 256 tiling, fp32 partials in a
 // workspace, an ordered reduction applying the epilogue): returns the split (0: none).
-uint32_t vsl_gemm_splitk_plan(uint32_t M, uint32_t N, uint32_t K, int epi, uint32_t min_items, uint64_t* ws_bytes);
+uint32_t vsl_gemm_splitk_plan(uint32_t M, uint32_t N, uint32_t K, int epi, int am, uint32_t min_items,
+                              uint64_t* ws_bytes);
 // The k-chunk partials alone, ws[chunk][M][N] fp32, for a caller that sums them itself.
 void vsl_gemm_splitk_partials(uint32_t ksplit, void* stream, const void* A, const void* B, uint32_t M, uint32_t N,
                               uint32_t K, int am, float* ws, int b8s);

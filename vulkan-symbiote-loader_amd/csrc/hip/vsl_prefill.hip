@@ -848,7 +848,7 @@ static uint32_t splitk_choice(uint32_t M, uint32_t N, uint32_t K, int epi, int a
         if (vsl_gemm_dma_tiles(cfg, M, N, K, epi) >= kDmaMinTiles) return 0;
     if (!ws) return 0;
     uint64_t need = 0;
-    const uint32_t ks = vsl_gemm_splitk_plan(M, N, K, epi, kDmaMinTiles, &need);
+    const uint32_t ks = vsl_gemm_splitk_plan(M, N, K, epi, am, kDmaMinTiles, &need);
     if (!ks || need > ws_bytes) return 0;
     const uint32_t rows = vsl_gemm_rows_split(M, N, K, am, ks);
     return rows ? rows : ks;
@@ -967,7 +967,7 @@ extern "C" int vsl_gemm_f16_direct(uint32_t M, uint32_t N, uint32_t K, int epilo
     const int epi = epilogue & 0xFF;
     for (int cfg = 0; cfg < 2; ++cfg)
         if (vsl_gemm_dma_tiles(cfg, M, N, K, epi) >= kDmaMinTiles) return 1;
-    return vsl_gemm_splitk_plan(M, N, K, epi, kDmaMinTiles, nullptr) ? 1 : 0;
+    return vsl_gemm_splitk_plan(M, N, K, epi, gemm_a_mode(epilogue), kDmaMinTiles, nullptr) ? 1 : 0;
 }
 
 extern "C" uint64_t vsl_gemm_f16_ws_bytes(uint32_t M, uint32_t N, uint32_t K, int epilogue) {
@@ -975,7 +975,7 @@ extern "C" uint64_t vsl_gemm_f16_ws_bytes(uint32_t M, uint32_t N, uint32_t K, in
     for (int cfg = 0; cfg < 2; ++cfg)
         if (vsl_gemm_dma_tiles(cfg, M, N, K, epi) >= kDmaMinTiles) return 0;
     uint64_t need = 0;
-    return vsl_gemm_splitk_plan(M, N, K, epi, kDmaMinTiles, &need) ? need : 0;
+    return vsl_gemm_splitk_plan(M, N, K, epi, gemm_a_mode(epilogue), kDmaMinTiles, &need) ? need : 0;
 }
 
 // RoPE + Q/K/V split of KS partials (KS = 1: the finished projection), four columns per thread.
