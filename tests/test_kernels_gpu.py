@@ -760,6 +760,35 @@ def test_lm_head_sampler_routes(vsl, orc, dev, H, V, mode, k):
     assert np.array_equal(dev.get(logits), l)
 
 
+@pytest.mark.parametrize("dt,V,d", [
+    ("F16", 9001, 64), ("F16", 8192, 8224), ("F16", 8200, 16416), ("F16", 3000, 16416),  # blocks of 4, 8 and 16 waves
+    ("F32", 8203, 16392), ("Q8_0", 9001, 64), ("Q8_0", 3000, 16416), ("Q4_0", 9001, 64), ("Q4_0", 3000, 8224),
+    ("Q4_1", 9001, 64), ("Q4_1", 3000, 16416),
+])
+def test_lm_head_sampler_row_maps(vsl, dev, H, dt, V, d):
+    """The samplers over the blocks' maxima know which rows each block of the projection took, over every
+    weight dtype and block size: the token is the one vsl_sample_logits draws from the logits written."""
+    rng = np.random.default_rng(V + d)
+    W = np.zeros((V, d), np.float32 if dt == "F32" else np.float16)
+    W[:, 0] = rng.normal(0, 1.3, V)
+    dtype, dW, nb = getattr(vsl, "VSL_DT_" + dt), dev.put(W), H.vsl_lm_head_ws_blocks()
+    if dt[0] == "Q":
+        pack = dev.empty((H.vsl_quant_pack_bytes(dtype, V, d),), np.uint8)
+        ok(vsl, H.vsl_quantize_pack(dev.p(dW), vsl.VSL_DT_F16, V, d, dtype, dev.p(pack), None))
+        dW = pack
+    x = np.zeros(d, np.float32)
+    x[0] = 1.0
+    ws_v, ws_i, out, toks = (dev.empty((n,), t) for n, t in ((nb, np.float32), (nb, np.int32), (1, np.int32), (1, np.int32)))
+    E, logits = dev.put(np.zeros((V, d), np.float16)), dev.empty((V,), np.float32)
+    for mode, k in ((2, 1), (2, 5), (2, 11), (2, 40), (2, 70), (1, 1)):
+        for seed in range(3):
+            smp, dx, c = vsl.Sampler(mode, 0.8, k, 0, seed), dev.put(x), ctrl_buf(vsl, dev, H, 3, max_steps=4, cap=64)
+            ok(vsl, H.vsl_lm_head_sample(None, 1e-5, dev.p(dW), dtype, V, d, dev.p(dx), dev.p(E), 1, dev.p(logits), smp,
+                                         dev.p(ws_v), dev.p(ws_i), dev.p(toks), dev.p(c), None))
+            ok(vsl, H.vsl_sample_logits(dev.p(logits), V, smp, 0, dev.p(out), None))
+            assert int(dev.get(toks)[0]) == int(dev.get(out)[0]), (mode, k, seed)
+
+
 @pytest.mark.parametrize("V,T", [(20000, 1.0), (128256, 1.0), (300000, 1.0), (9000, 0.7)])
 def test_lm_head_reference_near_ties(vsl, dev, H, V, T):
     """Reference mode picks the first index of the largest exp(l / T - max) / sum.  Two logits one ulp

@@ -622,10 +622,16 @@ uint32_t gemv_blocks(uint32_t N, uint32_t max_blocks) {
 
 constexpr uint32_t kMaxK = 32768;  // activation vector held in LDS as fp32 (up to 128 KB)
 
+// The row map of a launch: block b of `blocks` takes `rows` adjacent rows per pass over the grid.
+struct GemvGrid {
+    uint32_t blocks, rows;
+};
+
 // XPT: float4 of the activation vector staged per thread, the smallest power of two covering K
 template <class WT, int R, int U, int EPI, int WAVES, class ET = WF32>
-int launch_gemv(const GemvArgs& a, uint32_t max_blocks, hipStream_t s) {
+int launch_gemv(const GemvArgs& a, uint32_t max_blocks, hipStream_t s, GemvGrid* grid = nullptr) {
     const uint32_t blocks = gemv_blocks<R, EPI, WAVES>(a.N, max_blocks);
+    if (grid) *grid = {blocks, WAVES * (uint32_t)(EPI == EPI_SWIGLU ? R / 2 : R)};
     // the fp32 activation vector, and for 4-bit packs its 32-value block sums
     const size_t lds = (size_t)xs_floats(a.K) * sizeof(float) + (WT::kBits == 4 ? (size_t)a.K / 32 * sizeof(float) : 0);
     const uint32_t per = WAVES * 64 * 4;
@@ -666,17 +672,17 @@ uint32_t gemv_waves_k(uint32_t K) {
 }
 
 template <class WT, int R, int U, int EPI, class ET = WF32>
-int launch_gemv_k(const GemvArgs& a, uint32_t max_blocks, hipStream_t s) {
+int launch_gemv_k(const GemvArgs& a, uint32_t max_blocks, hipStream_t s, GemvGrid* grid = nullptr) {
     switch (gemv_waves_k(a.K)) {
-        case 16: return launch_gemv<WT, R, U, EPI, 16, ET>(a, max_blocks, s);
-        case 8: return launch_gemv<WT, R, U, EPI, 8, ET>(a, max_blocks, s);
-        default: return launch_gemv<WT, R, U, EPI, 4, ET>(a, max_blocks, s);
+        case 16: return launch_gemv<WT, R, U, EPI, 16, ET>(a, max_blocks, s, grid);
+        case 8: return launch_gemv<WT, R, U, EPI, 8, ET>(a, max_blocks, s, grid);
+        default: return launch_gemv<WT, R, U, EPI, 4, ET>(a, max_blocks, s, grid);
     }
 }
 
 template <int R, int EPI>
 uint32_t gemv_blocks_k(uint32_t N, uint32_t K, uint32_t max_blocks) {
-    // the grid launch_gemv_k chooses
+    // the grid launch_gemv_k chooses (for rules taken before the launch)
     switch (gemv_waves_k(K)) {
         case 16: return gemv_blocks<R, EPI, 16>(N, max_blocks);
         case 8: return gemv_blocks<R, EPI, 8>(N, max_blocks);
@@ -705,40 +711,41 @@ bool quant_dtype(int wdtype) { return wdtype == VSL_DT_Q8_0 || wdtype == VSL_DT_
 // 70B-class down projection (8192 rows) 30.5 -> 28.0 us, O 11.3 -> 11.1 us; with 4096 rows (8B: half
 // the waves idle) 10.4 -> 13.4 / 13.6 -> 17.4 us, so only from 8192 rows.
 template <class WT, int R, int U, int EPI, class ET>
-int launch_gemv_q(const GemvArgs& a, uint32_t max_blocks, hipStream_t s) {
+int launch_gemv_q(const GemvArgs& a, uint32_t max_blocks, hipStream_t s, GemvGrid* grid = nullptr) {
     if (gemv_waves_env() == 0) {
         if constexpr (EPI == EPI_SWIGLU) {
-            if (a.K <= kXWideK) return launch_gemv<WT, R, U, EPI, 8, ET>(a, max_blocks, s);
+            if (a.K <= kXWideK) return launch_gemv<WT, R, U, EPI, 8, ET>(a, max_blocks, s, grid);
         } else if constexpr (EPI == EPI_RESID) {
             if (a.K >= kWideK) {
                 // two rows per wave once the rows fill every resident wave twice over (each staged
                 // activation read then serves two rows)
                 if constexpr (R == 1) {
                     if ((uint64_t)a.N >= 2ull * 16ull * gemv_grid_cap(16, EPI_RESID))
-                        return launch_gemv<WT, 2, U, EPI, 16, ET>(a, max_blocks, s);
+                        return launch_gemv<WT, 2, U, EPI, 16, ET>(a, max_blocks, s, grid);
                 }
-                return launch_gemv<WT, R, U, EPI, 16, ET>(a, max_blocks, s);
+                return launch_gemv<WT, R, U, EPI, 16, ET>(a, max_blocks, s, grid);
             }
         }
     }
-    return launch_gemv_k<WT, R, U, EPI, ET>(a, max_blocks, s);
+    return launch_gemv_k<WT, R, U, EPI, ET>(a, max_blocks, s, grid);
 }
 
 // The decode GEMV over the weight dtype: fp16 / fp32 matrices with four 16-byte loads per lane and row
 // per tile; block-quantized packs with the same 2048 columns per tile (Q8: two loads of 16 values,
 // Q4: one of 32).
 template <int R, int EPI, class ET = WF32>
-int launch_gemv_w(int wdtype, const GemvArgs& a, uint32_t max_blocks, hipStream_t s, const char* who) {
+int launch_gemv_w(int wdtype, const GemvArgs& a, uint32_t max_blocks, hipStream_t s, const char* who,
+                  GemvGrid* grid = nullptr) {
     if (quant_dtype(wdtype)) {
         if (a.K % 32) return vsl_invalid("%s: a block-quantized pack needs K %% 32 == 0 (K=%u)", who, a.K);
         if (reinterpret_cast<uintptr_t>(a.W) & 255) return vsl_invalid("%s: a block-quantized pack must be 256-byte aligned", who);
     }
     switch (wdtype) {
-        case VSL_DT_F16: return launch_gemv_k<WF16, R, 4, EPI, ET>(a, max_blocks, s);
-        case VSL_DT_F32: return launch_gemv_k<WF32, R, 4, EPI, ET>(a, max_blocks, s);
-        case VSL_DT_Q8_0: return launch_gemv_q<WQ8, R, 2, EPI, ET>(a, max_blocks, s);
-        case VSL_DT_Q4_0: return launch_gemv_q<WQ4, R, 1, EPI, ET>(a, max_blocks, s);
-        case VSL_DT_Q4_1: return launch_gemv_q<WQ41, R, 1, EPI, ET>(a, max_blocks, s);
+        case VSL_DT_F16: return launch_gemv_k<WF16, R, 4, EPI, ET>(a, max_blocks, s, grid);
+        case VSL_DT_F32: return launch_gemv_k<WF32, R, 4, EPI, ET>(a, max_blocks, s, grid);
+        case VSL_DT_Q8_0: return launch_gemv_q<WQ8, R, 2, EPI, ET>(a, max_blocks, s, grid);
+        case VSL_DT_Q4_0: return launch_gemv_q<WQ4, R, 1, EPI, ET>(a, max_blocks, s, grid);
+        case VSL_DT_Q4_1: return launch_gemv_q<WQ41, R, 1, EPI, ET>(a, max_blocks, s, grid);
         default: return vsl_unsupported("%s: weight dtype %d", who, wdtype);
     }
 }
@@ -3043,25 +3050,25 @@ extern "C" int vsl_lm_head_sample(const float* gamma, float eps, const void* W, 
     a.W = W; a.N = V; a.K = d; a.x = x; a.gamma = gamma; a.eps = eps; a.y = logits;
     a.ws_val = ws_val; a.ws_idx = ws_idx; a.tokens = tokens; a.embed = embed; a.x_next = x;
     a.ctrl = ctrl;
-    const uint32_t nb = gemv_blocks_k<2, EPI_ARGMAX>(V, d, kMaxLmBlocks);
-    const bool maxima = fused || use_block_maxima(sampler, V, nb);
-    if (int rc = maxima ? launch_gemv_w<2, EPI_ARGMAX>(wdtype, a, kMaxLmBlocks, s, "vsl_lm_head_sample")
+    const bool maxima = fused || use_block_maxima(sampler, V, gemv_blocks_k<2, EPI_ARGMAX>(V, d, kMaxLmBlocks));
+    GemvGrid grid{};  // whatever shape the projection takes, the samplers read its maxima by the map it ran with
+    if (int rc = maxima ? launch_gemv_w<2, EPI_ARGMAX>(wdtype, a, kMaxLmBlocks, s, "vsl_lm_head_sample", &grid)
                         : launch_gemv_w<2, EPI_STORE>(wdtype, a, 1u << 20, s, "vsl_lm_head_sample"))
         return rc;
     if (fused) {
         if (embed_dtype == VSL_DT_F16)
-            k_argmax_finish<WF16><<<1, kFinishThreads, 0, s>>>(ws_val, ws_idx, nb, V, d, embed, x, tokens, ctrl);
+            k_argmax_finish<WF16><<<1, kFinishThreads, 0, s>>>(ws_val, ws_idx, grid.blocks, V, d, embed, x, tokens, ctrl);
         else
-            k_argmax_finish<WF32><<<1, kFinishThreads, 0, s>>>(ws_val, ws_idx, nb, V, d, embed, x, tokens, ctrl);
+            k_argmax_finish<WF32><<<1, kFinishThreads, 0, s>>>(ws_val, ws_idx, grid.blocks, V, d, embed, x, tokens, ctrl);
         HIP_TRY(hipGetLastError());
         return VSL_OK;
     }
     const uint64_t key = vsl_derive_key(sampler.seed, "sampler");
     float* part = reinterpret_cast<float*>(ws_idx);
-    LmBlocks lb{ws_val, part, nb, 0};
-    while ((1u << lb.rpb_log2) < 2 * gemv_waves_k(d)) ++lb.rpb_log2;  // two rows per wave
+    LmBlocks lb{ws_val, part, grid.blocks, 0};
+    while ((1u << lb.rpb_log2) < grid.rows) ++lb.rpb_log2;  // waves x rows per wave: a power of two
     if (sampler.mode == VSL_SAMPLE_REFERENCE && maxima) {
-        k_reference_sum<<<kRefBlocks, kRefThreads, 0, s>>>(logits, V, sampler.temperature, ws_val, nb, part, ctrl);
+        k_reference_sum<<<kRefBlocks, kRefThreads, 0, s>>>(logits, V, sampler.temperature, ws_val, grid.blocks, part, ctrl);
         HIP_TRY(hipGetLastError());
     }
     auto finish = [&](auto kernel) {
