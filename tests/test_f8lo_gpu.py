@@ -220,6 +220,8 @@ def test_gemm_mixed_rounds(vsl, dev, H, M, N, K, amode):
     (512, 6144, 4096, 0),    # 8B QKV (128 x 192 tiles)
     (128, 2048, 8192, 2),    # 1B down projection of a 128-row prompt: 32 chunks
     (300, 4096, 2048, 1),    # ragged M, fp16 store
+    (700, 6144, 4096, 0),    # one chunk: 192 tiles of 128 x 192
+    (1274, 4096, 14336, 2),  # two chunks of 160 tiles
 ])
 def test_gemm_f8lo_splitk(vsl, dev, H, M, N, K, epi):
     """Narrow shapes split over K with an F16F8 A: the partials come from the fp8 lo path of the
@@ -251,8 +253,8 @@ def test_gemm_f8lo_splitk(vsl, dev, H, M, N, K, epi):
 
 
 @pytest.mark.parametrize("M,N,K,epi,amode,cmode", [
-    (1, 6144, 512, 0, "x2", None),      # 96 weight rows per block, two chunks, one unit per wave
-    (3, 6144, 4096, 0, "f8", None),     # 8B QKV
+    (1, 6144, 512, 0, "x2", None),      # 64 weight rows per block, two chunks, one unit per wave
+    (3, 6144, 4096, 0, "f8", None),     # 8B QKV: 96 weight rows per block
     (17, 2048, 2048, 2, "x2", None),    # 64 weight rows per block, residual add
     (45, 4096, 4096, 2, "f8", None),    # 8B O projection: 128 weight rows per block
     (64, 4096, 14336, 2, "x2", None),   # 8B down projection, seven units per wave
@@ -320,6 +322,32 @@ def test_gemm_few_rows(vsl, dev, H, M, N, K, epi, amode, cmode):
         assert rel_err(out, prod) < 2.0 ** -10
     else:
         assert rel_err(out - (C0 if epi == 2 else 0.0), prod) < 5e-6
+
+
+@pytest.mark.parametrize("epi,amode", [(0, "f8"), (0, "x2"), (1, "x2"), (2, "f8"), (2, "x2")])
+def test_gemm_mixed_rounds_stores(vsl, dev, H, epi, amode):
+    """The fp32-store, fp16-store and residual products of 1540 rows and 10240 outputs (a 70B-class QKV): 36
+    columns of 256 x 256 tiles, the last 4 on 128 x 256 ones."""
+    M, N, K = 1540, 10240, 256
+    rng = np.random.default_rng(epi + len(amode))
+    A, B = rng.normal(0, 1, (M, K)).astype(np.float32), rng.normal(0, 0.02, (N, K)).astype(np.float16)
+    rows = np.unique(np.concatenate([[0, 127, 128, 255, 256, 1535, 1536, M - 1], rng.integers(0, M, 24)]))
+    if amode == "f8":
+        dA, hi, val = f8_buffer(dev, A)
+        ref = T.f8lo_product(hi[rows], val[rows] - hi[rows].astype(np.float64), B)
+    else:
+        hi = A.astype(np.float16)
+        lo = (A - hi.astype(np.float32)).astype(np.float16)
+        dA = dev.put(np.concatenate([hi, lo]))
+        ref = (hi[rows].astype(np.float64) + lo[rows].astype(np.float64)) @ B.astype(np.float64).T
+    C0 = rng.normal(0, 1, (M, N)).astype(np.float16 if epi == 1 else np.float32)
+    C = dev.put(C0)
+    ok(vsl, H.vsl_gemm_f16(dev.p(dA), dev.p(dev.put(B)), M, N, K, dev.p(C),
+                           epi | (vsl.GEMM_A_F8 if amode == "f8" else vsl.GEMM_A_X2), None))
+    out = dev.get(C).astype(np.float64)[rows]
+    if epi == 2:  # both the product and the stored sum round to fp32
+        ref = ref + C0[rows].astype(np.float64)
+    assert rel_err(out, ref) < (2.0 ** -10 if epi == 1 else 5e-6)
 
 
 @pytest.mark.parametrize("n,off", [(1, 0), (7, 0), (8, 0), (1000, 1), (4097, 3), (1 << 20, 0), ((1 << 20) + 5, 8)])
@@ -465,7 +493,7 @@ def test_gemm_f8lo_forms_refused(vsl, dev, H):
     assert H.vsl_gemm_f16(dev.p(A), dev.p(B), 64, 4096, 4096, dev.p(C), vsl.GEMM_C_F8, None) == vsl.VSL_E_INVALID
 
 
-@pytest.mark.parametrize("M,N,K", [(512, 4096, 14336), (300, 2048, 8192)])
+@pytest.mark.parametrize("M,N,K", [(512, 4096, 14336), (300, 2048, 8192), (1400, 4096, 4096)])  # the last: one chunk
 def test_resid_rmsnorm_f8lo(vsl, orc, dev, H, M, N, K):
     """The down projection's entry with an F16F8 input and an F16F8 normalized output: the fused launch
     (K split) leaves x exactly as the unfused residual GEMM does, and both it and the unsplit path

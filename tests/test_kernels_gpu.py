@@ -128,9 +128,9 @@ def test_gemv_batched_rows(vsl, orc, dev, H, N, K, B, ydt):
 @pytest.mark.parametrize("N,K,B,ydt,off", [
     (1, 512, 2, 0, 0),         # one row; eight units for the 16-wave blocks
     (300, 1536, 5, 1, 0),      # a ragged last fragment, odd B
-    (6143, 2048, 16, 0, 0),    # the largest N of one fragment per block
-    (6144, 512, 3, 1, 0), (12271, 1024, 7, 0, 0),     # two fragments: one unit per wave; ragged end
-    (12272, 512, 16, 0, 0), (14337, 1536, 9, 1, 0),   # four fragments: two units; six; ragged end
+    (6128, 2048, 16, 0, 0),    # the largest N of one fragment per block
+    (6129, 512, 3, 1, 0), (12271, 1024, 7, 0, 0), (12272, 512, 5, 0, 0),   # two fragments: one unit per wave; two; one
+    (12273, 512, 16, 0, 0), (14337, 1536, 9, 1, 0),   # four fragments: two units per wave; six; ragged ends
     (1000, 14336, 4, 0, 0),    # fourteen units per wave
     (500, 1024, 6, 0, 1),      # X not 16-byte aligned: the gathering kernel
 ])
@@ -917,9 +917,14 @@ def test_gemm_dma(vsl, orc, dev, H, M, N, K, epi, ax2, cx2):
     (300, 6144, 4096, 2, True),    # ragged M on 128 x 192 tiles, residual add
     (512, 4096, 4096, 1, False),   # fp16 store
     (300, 4096, 2048, 2, False),   # ragged M
-    (128, 2048, 8192, 2, True),    # 1B down projection of a 128-row prompt: 32 chunks of 256
-    (128, 3072, 2048, 0, True),    # 1B QKV: 16 chunks of 128 reach 192 items
+    (128, 2048, 8192, 2, True),    # 1B down projection of a 128-row prompt: few-row kernel, 8 chunks
+    (128, 3072, 2048, 0, True),    # 1B QKV: few-row kernel, 4 chunks
+    (128, 2048, 8192, 2, False),   # the same two of one-plane A: 32 chunks of 256,
+    (128, 3072, 2048, 0, False),   # 16 chunks of 128 on 128 x 192 tiles
     (128, 2048, 2048, 2, False),   # 1B O projection: the widest split (16) short of 192 items
+    (700, 6144, 4096, 0, True),    # one chunk: 192 tiles of 128 x 192
+    (1400, 4096, 4096, 2, False),  # one chunk: 176 tiles of 128 x 256, one-plane A
+    (1146, 2048, 14336, 2, True),  # two chunks of 72 tiles, 7168 columns each
 ])
 def test_gemm_splitk(vsl, dev, H, M, N, K, epi, ax2):
     """Narrow shapes through vsl_gemm_f16_ws: split over K into a workspace (128 x 256 tiles, or 128 x 192
@@ -1242,9 +1247,12 @@ def _act(rng, M, K, ax2):
 @pytest.mark.parametrize("S,K,nq,nkv,hd,pos0,ax2,qx2,kvdt", [
     (512, 4096, 32, 8, 128, 0, True, True, 1),     # 512-row chunk of the 8B-class model: K split 2
     (512, 4096, 32, 8, 128, 100, False, False, 1),  # later chunk, fp16 q
-    (300, 4096, 32, 8, 128, 7, True, True, 0),     # ragged rows (K split 4), fp32 cache
+    (300, 4096, 32, 8, 128, 7, True, True, 0),     # ragged rows, fp32 cache
     (256, 4096, 32, 8, 64, 0, False, True, 1),     # head_dim 64 (K split 8)
-    (128, 2048, 32, 8, 64, 0, True, True, 1),      # 1B 128-row prompt: K split 16 (runtime-count sum)
+    (128, 2048, 32, 8, 64, 0, True, True, 1),      # 1B 128-row prompt: few-row kernel, K split 4
+    (128, 2048, 32, 8, 64, 5, False, True, 1),     # the same of one-plane A: K split 16 (runtime-count sum)
+    (700, 4096, 32, 8, 128, 3, True, True, 1),     # one chunk (runtime-count sum of one)
+    (64, 4096, 32, 8, 128, 9, True, False, 0),     # few-row kernel, K split 4, fp16 q, fp32 cache
 ])
 def test_gemm_qkv_rope_append(vsl, orc, dev, H, S, K, nq, nkv, hd, pos0, ax2, qx2, kvdt):
     """QKV projection + RoPE + Q/K/V split through one entry point. With the workspace the split-K
@@ -1324,8 +1332,10 @@ def test_gemm_qkv_rope_append_refuses_before_launch(vsl, dev, H):
     (300, 4096, 4096, False, 1, True),   # ragged rows, fp16 out
     (512, 2048, 8192, False, 0, False),  # d = 2048, K split 8, fp32 out, no gains
     (256, 8192, 4096, False, 2, True),   # d = 8192 (eight float4 per thread)
-    (128, 2048, 8192, True, 2, True),    # 1B down projection of a 128-row prompt: K split 32
+    (128, 2048, 8192, True, 2, True),    # 1B down projection of a 128-row prompt: few-row kernel, K split 8
+    (128, 2048, 8192, False, 2, True),   # the same of one-plane A: K split 32
     (128, 2048, 2048, False, 1, True),   # 1B O projection: K split 16
+    (1400, 4096, 4096, True, 2, True),   # one chunk: 176 tiles
 ])
 def test_gemm_resid_rmsnorm(vsl, orc, dev, H, M, N, K, ax2, odt, gam):
     """Residual projection + the next RMSNorm through one entry point. With the workspace the split-K

@@ -10,7 +10,7 @@
 // waves' sums meet. Block = 16 NF rows of W; its WAVES waves take every WAVES-th 64-column unit of K, and
 // the 16 NF rows share each X unit: NF = 4 where that still gives three quarters of the CUs a block, else 2
 // or 1 with as many more waves. The weights of the wide blocks are loaded non-temporally; those of one
-// fragment per block are small matrices (up to 6143 rows) that a repeated product finds in the cache. The
+// fragment per block are small matrices (up to 6128 rows) that a repeated product finds in the cache. The
 // blocks of an XCD start at different units, three apart: rows of a power-of-two stride put one unit of
 // all rows on few memory channels.
 // N x K, B (gathering kernel -> this one, us): 14336 x 4096, 16 30.5 -> 18.9; 4096 x 4096, 9 8.3 -> 7.1;
