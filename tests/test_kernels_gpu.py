@@ -126,7 +126,8 @@ def test_gemv_batched_rows(vsl, orc, dev, H, N, K, B, ydt):
 
 
 @pytest.mark.parametrize("N,K,B,ydt,off", [
-    (1, 512, 2, 0, 0),         # one row; eight units for the 16-wave blocks
+    (1, 512, 2, 0, 0), (6128, 512, 3, 1, 0),          # 512 columns of one fragment: the gathering kernel
+    (1, 1024, 2, 0, 0),        # one row, one unit per wave
     (300, 1536, 5, 1, 0),      # a ragged last fragment, odd B
     (6128, 2048, 16, 0, 0),    # the largest N of one fragment per block
     (6129, 512, 3, 1, 0), (12271, 1024, 7, 0, 0), (12272, 512, 5, 0, 0),   # two fragments: one unit per wave; two; one

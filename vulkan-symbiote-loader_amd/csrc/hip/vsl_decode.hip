@@ -2288,7 +2288,7 @@ constexpr uint32_t kSkKAlign = kSkWaves * 32 * kSkU * 2;  // K multiple: whole g
 // VEC_MAJOR: X holds B vectors of K ([B][K]) and Y B vectors of N ([B][N]) -- a batch of
 // activation vectors, each contiguous -- so a lane's X operand is one 16-byte load; otherwise X is
 // [K][B] and Y [N][B] (row-major products), eight 2-byte loads per operand. That form only serves an X
-// that is not 16-byte aligned (vsl_skinny.hip the others).
+// that is not 16-byte aligned and few rows of 512 columns (vsl_skinny.hip the others).
 template <typename YT, bool VEC_MAJOR, int R>
 __global__ __launch_bounds__(kSkWaves * 64) void k_skinny(const vsl_half* __restrict__ W, uint32_t N, uint32_t K,
                                                          const vsl_half* __restrict__ X, uint32_t B, YT* __restrict__ Y) {
@@ -2803,13 +2803,15 @@ extern "C" int vsl_gemv(const void* W, int wdtype, uint32_t N, uint32_t K, const
     if (wdtype == VSL_DT_F16 && xdtype == VSL_DT_F16 && B == 1 && K % 8 == 0 && K <= kMaxK &&
         (reinterpret_cast<uintptr_t>(X) & 7) == 0)
         return gemv_one_f16x(W, N, K, X, Y, ydtype, s);
+    // (at K = 512 half of the 16 waves of vsl_skinny.hip's one-fragment blocks have no unit: 4096 x 512, 16 2.59 us
+    // gathering / 2.72, 256 x 512, 4 2.35 / 2.45; from 1024 columns it is faster, 256 x 1024, 4 3.00 / 2.85)
     if (wdtype == VSL_DT_F16 && xdtype == VSL_DT_F16 && K % kSkKAlign == 0 && B > 1 &&
-        (reinterpret_cast<uintptr_t>(X) & 15) == 0) {
+        (K > 512 || N > kSkinnyOneFragN) && (reinterpret_cast<uintptr_t>(X) & 15) == 0) {
         vsl_skinny_rows(W, N, K, X, B, Y, ydtype == VSL_DT_F16, stream);
         HIP_TRY(hipGetLastError());
         return VSL_OK;
     }
-    // an X that is not 16-byte aligned
+    // few rows of 512 columns, or an X that is not 16-byte aligned
     if (wdtype == VSL_DT_F16 && xdtype == VSL_DT_F16 && K % kSkKAlign == 0)
         return ydtype == VSL_DT_F16 ? launch_skinny<vsl_half, false>(W, N, K, X, B, Y, s)
                                     : launch_skinny<float, false>(W, N, K, X, B, Y, s);

@@ -10,13 +10,15 @@
 // waves' sums meet. Block = 16 NF rows of W; its WAVES waves take every WAVES-th 64-column unit of K, and
 // the 16 NF rows share each X unit: NF = 4 where that still gives three quarters of the CUs a block, else 2
 // or 1 with as many more waves. The weights of the wide blocks are loaded non-temporally; those of one
-// fragment per block are small matrices (up to 6128 rows) that a repeated product finds in the cache. The
+// fragment per block (up to 6128 rows) are not: a product repeated over one such matrix finds it in the cache,
+// while matrices that come from memory each time lose (plain / non-temporal, us, repeated: 4096 x 4096, 16 6.6 /
+// 7.0, 4096 x 14336, 16 19.9 / 22.4; from memory: 8.8 / 8.4, 25.0 / 23.2; both under the gathering kernel's). The
 // blocks of an XCD start at different units, three apart: rows of a power-of-two stride put one unit of
 // all rows on few memory channels.
-// N x K, B (gathering kernel -> this one, us): 14336 x 4096, 16 30.5 -> 18.9; 4096 x 4096, 9 8.3 -> 7.1;
-// 1000 x 14336, 4 21.2 -> 12.9; 32000 x 2048, 16 35.2 -> 22.1; 8000 x 8192, 12 37.8 -> 24.8. (Weights loaded in the
-// operand layout, 64 bytes of each of 16 rows: 22.4, 7.3, 17.3, 25.3, 27.9; non-temporal for all: 19.0, 8.1, 15.1,
-// 22.1, 24.1; every block starting at the same unit: 26.1 in the operand layout for the first shape.)
+// N x K, B (gathering kernel -> this one, us; one matrix repeated | matrices from memory): 14336 x 4096, 16
+// 23.5 -> 19.4 | 30.4 -> 20.2; 4096 x 4096, 9 8.0 -> 6.4 | 10.6 -> 8.5; 1000 x 14336, 4 20.4 -> 12.8 | 28.7 -> 15.9;
+// 32000 x 2048, 16 24.8 -> 21.3 | 32.7 -> 21.8; 8000 x 8192, 12 25.9 -> 23.2 | 34.5 -> 24.0 (graphs of one product after
+// another).
 #include <hip/hip_runtime.h>
 
 #include "vsl_device.h"
@@ -26,6 +28,7 @@ namespace {
 
 constexpr uint32_t kUnit = 64;     // columns of K per wave step
 constexpr uint32_t kSkinnyCUs = 256;  // MI355X compute units
+static_assert(kSkinnyOneFragN == (3 * kSkinnyCUs / 2 - 1) * 16, "two fragments per block from three quarters of the CUs");
 
 template <int NF, int WAVES, typename YT>
 __global__ __launch_bounds__(WAVES * 64) void k_skinny_rows(const vsl_half* __restrict__ W, uint32_t N, uint32_t K,
@@ -132,7 +135,7 @@ template <typename YT>
 void launch(const vsl_half* w, uint32_t N, uint32_t K, const vsl_half* x, uint32_t B, YT* y, hipStream_t s) {
     const uint32_t frags = (N + 15) / 16;
     if (frags >= 3 * kSkinnyCUs) k_skinny_rows<4, 4, YT><<<(frags + 3) / 4, 256, 0, s>>>(w, N, K, x, B, y);
-    else if (frags >= 3 * kSkinnyCUs / 2) k_skinny_rows<2, 8, YT><<<(frags + 1) / 2, 512, 0, s>>>(w, N, K, x, B, y);
+    else if (N > kSkinnyOneFragN) k_skinny_rows<2, 8, YT><<<(frags + 1) / 2, 512, 0, s>>>(w, N, K, x, B, y);
     else k_skinny_rows<1, 16, YT><<<frags, 1024, 0, s>>>(w, N, K, x, B, y);
 }
 
