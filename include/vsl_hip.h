@@ -320,6 +320,10 @@ int vsl_ctrl_reset(vsl_ctrl* ctrl, uint32_t pos, uint32_t max_steps, uint32_t st
  * plane on fp16 MFMA, the lo plane on fp8 MFMA against B rounded to e4m3 as B * 2^s, into the same
  * fp32 accumulators), VSL_GEMM_C_F8 (SwiGLU output written as VSL_DT_F16F8).  The F8 forms need
  * N % 256 == 0 (N % 128 == 0 for SwiGLU) and K % 128 == 0, else VSL_E_UNSUPPORTED.
+ * Up to 64 rows of 16-byte-aligned operands the F8 form's lo plane is widened to fp16 exactly and
+ * multiplied by the fp16 weights themselves (the few-row kernel; the weight shift is checked and not
+ * used), so a row's product is closer to the carried value there than in a larger chunk, by up to the
+ * weights' e4m3 rounding of a lo plane 2^-11 of the hi plane.
  * The weight shift s of the fp8 lo product is or'ed in as VSL_GEMM_B8_SHIFT(s), -16 <= s <= 30
  * (without it s = 6).  e4m3 holds magnitudes up to 448 and the conversion does not saturate, so
  * every |B| * 2^s must be <= 448: vsl_gemm_b8_shift gives the largest such s for a matrix's

@@ -569,10 +569,11 @@ void launch_splitk(uint32_t items, hipStream_t s, const vsl_half* a, const vsl_h
 }
 
 // Whole rounds of 256 x 256 tiles, the rest of the columns on 128 x 256 tiles: the columns for the first,
-// or all of them where that costs no less. A 128 x 256 tile takes ~0.6 of a 256 x 256 one (fp8-lo, K =
-// 4096: 108 against 180 us a round of 256), so a last round less than half full is halved instead of
-// left idle: the layer's prompt pass of 8B at 2048 rows (896 gate/up tiles, 3.5 rounds) 1950 -> 1915 us, 700
-// rows (336 tiles) 689 -> 643, 1200 rows 1092 -> 1044. (One-plane A, whose ratio differs, keeps whole tiles.)
+// or all of them where the rest would not fit one round. A 128 x 256 tile takes ~0.6 of a 256 x 256 one
+// (fp8-lo, K = 4096: 108 against 180 us a round of 256), so a last round less than half full is halved instead
+// of left idle: 8B gate/up (fp8 lo) of 2048 rows (896 tiles, 3.5 rounds) 697 -> 642 us, of 700 rows (336 tiles) 322
+// -> 271. Both split forms gained at every shape measured (K 1024 to 28672, SwiGLU and fp32 store, 2.7 to
+// 18 %); one-plane A was not and keeps whole tiles.
 template <int EPI>
 uint32_t big_columns(uint32_t M, uint32_t N) {
     constexpr uint32_t kCUs = 256;
@@ -581,7 +582,7 @@ uint32_t big_columns(uint32_t M, uint32_t N) {
     if (!full || tiles % kCUs == 0) return cols;
     const uint32_t big = full * kCUs / n_m;
     const uint32_t rest = ((cols - big) * n_m2 + kCUs - 1) / kCUs;
-    return big && 0.6 * rest < 0.9 ? big : cols;
+    return big && rest == 1 ? big : cols;
 }
 
 template <int EPI>

@@ -5,22 +5,23 @@
 // HBM-bound: at M = 45 a 28672 x 4096 product moves 235 MB of weights for 21 GFLOP of matrix work. The
 // tiles of the general kernels (vsl_gemm_dma.hip) pad such a chunk to 64 or 128 rows, carry the padding
 // through L2 and LDS, and meet at a block barrier every 64 columns. Here the waves share nothing inside
-// the main loop: a block owns 16 NF weight rows, its four waves (one per SIMD, up to 512 registers each)
-// take every fourth 64-column unit of K, load its weight and activation rows by whole 128-byte lines
-// one unit ahead, and turn each unit into v_mfma_f32_16x16x32_f16 operands in LDS of their own. The
-// waves' sums meet once, in wave order. The activations are re-read per block, from L2 (16 MT rows x 2
-// planes against 16 NF weight rows): loads of eight whole lines fetch them at 18 TB/s, loads in the
-// operand layout (64 bytes of each of 16 rows, adjacent lanes in different rows) at 8 TB/s.
+// the main loop: a block owns 16 NF weight rows, its four waves (one per SIMD, up to 512 registers each;
+// eight where a block has one fragment and at most 32 activation rows) take every fourth (eighth)
+// 64-column unit of K, load its weight and activation rows by whole 128-byte lines one unit ahead, and turn
+// each unit into v_mfma_f32_16x16x32_f16 operands in LDS of their own. The waves' sums meet once, in wave
+// order. The activations are re-read per block, from L2 (16 MT rows x 2 planes against 16 NF weight rows):
+// loads of eight whole lines fetch them at 18 TB/s, loads in the operand layout (64 bytes of each of 16
+// rows, adjacent lanes in different rows) at 8 TB/s.
 //
-// The weights of the wide blocks are loaded non-temporally, each line once (8B layer of 45 rows 140.6 -> 133.4
-// us, of 3 rows 117.0 -> 105.3); the narrow shapes' (NF = 1) are small and keep plain loads (45.0 against 47.1).
+// The weights of the wide blocks are loaded non-temporally (8B layer of 45 rows 140.6 -> 133.4 us, of 3 rows
+// 117.0 -> 105.3). With two row blocks (65 to 128 rows) each line is read twice and not kept between (1B down
+// of 128 rows fetches 77.7 MB for 33.6 MB of weights); plain loads are level there, weights from memory, us, plain
+// / non-temporal: 3072 x 2048 of 128 rows 15.4 / 15.4, 2048 x 8192 25.0 / 24.8, 8192 x 2048 23.7 / 22.4, 2048 x
+// 14336 33.6 / 34.5. The narrow shapes' weights (NF = 1) are small and keep plain loads (45.0 against 47.1).
 //
 // A layer's prompt pass, before (the tiles of vsl_gemm_dma.hip) -> with this kernel, us: 8B 45 rows 170.3 ->
 // 133.4, 3 rows 158.6 -> 105.3, 64 rows 177.5 -> 149.4; 1B 45 rows 99.2 -> 76.3, 7 rows 89.3 -> 61.8, 128 rows
-// 108.1 -> 96.8; 70B 40 rows 624.6 -> 357.0; d 768 with 30 rows 88.6 -> 45.0. Also measured at 45 / 64 rows of the 8B
-// layer, all with plain loads (this kernel 142.8 / 161.2): both operands in the operand layout 156 / 181; the
-// weights alone in it 144 / 171; two register sets ahead instead of one 149 / 218 (the second set's copies
-// and spills); eight waves of 32-column units 159 / 184.
+// 108.1 -> 96.8; 70B 40 rows 624.6 -> 357.0; d 768 with 30 rows 88.6 -> 45.0.
 #include <hip/hip_runtime.h>
 
 #include "vsl_device.h"
@@ -295,8 +296,10 @@ struct RowsPlan {
 // (4 x 16 rows everywhere: 8B layer of 45 rows 143 -> 171-188 us, of 3 rows 117 -> 133). More than 64 rows
 // run as two row blocks that share their weights through L2, in one round of blocks and for the narrow
 // models' products only (N or K up to 2048: the 1B layer's QKV of 128 rows 22.4 -> 15.8 us, O 22.1 -> 15.6,
-// down 27.7 -> 25.5); past that the activations read by every block outweigh what the general tiles waste (8B layer
-// of 100 rows 206.9 -> 215.9 with them, and 236 where gate/up took two rounds).
+// down 27.7 -> 25.5); past that the activations read by every block outweigh what the general tiles
+// waste (5120 x 3072 of 96 rows 22.1 -> 31.6, 6144 x 4096 25.6 either way, 4096 x 14336 45.7 -> 50.4, 5120 x 5120
+// 40.8 -> 53.1). Widths of 2304 to 3072 on both sides and 4096 x 4096 would gain (2560 x 2560 of 96 rows 38.9 ->
+// 22.5, 3072 x 3072 27.8 -> 23.8, 4096 x 4096 27.3 -> 23.1) and are not served.
 RowsPlan rows_plan(uint32_t M, uint32_t N, uint32_t K, bool sw, int am, uint32_t max_ks) {
     RowsPlan best;
     const uint64_t brows = sw ? 2ull * N : N;
