@@ -635,7 +635,7 @@ static bool splitk_narrow(uint32_t M, uint32_t N, uint32_t ksplit) {
 // the rounds of 256 blocks (product with its residual + RMSNorm or store, us: 1B O of 600 rows, 40 tiles, 8
 // -> 4 chunks 32.6 -> 26.8; 1B QKV of 700 rows 38.7 -> 30.6), down to one chunk where its tiles still fill five
 // eighths of the CUs (8B O of 1400 rows, 176 tiles, 131.3 -> 113.5; 1100 rows, 144 tiles, stay at two). The
-// hi/lo form gains over all shapes measured (N 1536 to 10240, K 1536 to 28672). The others, whose blocks are
+// hi/lo form gains over the shapes measured (N 1536 to 10240, K 1536 to 28672) but one. The others, whose blocks are
 // shorter, lose with long chunks where
 // - the narrow one-plane tiles (80 KB of LDS) no longer run two to a CU: 3072 x 14336 of 1530 rows one chunk
 //   +17 %, of 762 rows two +8 %, 9216 x 4096 of 506 rows -3 %, 3072 x 2048 of 1530 rows -3 %;
